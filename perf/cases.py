@@ -95,6 +95,16 @@ def draw(rng):
 
 # ---- inputs ------------------------------------------------------------------
 
+_streams = []
+
+
+def _stream():
+    """The program's one stream: a pass starts when the one before it has ended."""
+    if not _streams:
+        _streams.append(torch.cuda.Stream())
+    return _streams[0]
+
+
 def _gen(seed):
     g = torch.Generator(device="cuda")
     g.manual_seed(int(seed) % (1 << 62))
@@ -269,7 +279,7 @@ def _tokens(c, seed):
 def prepare(case, seed):
     c, s = case, _State()
     s.case, kind = c, c["kind"]
-    s.stream = torch.cuda.Stream()
+    s.stream = _stream()
     if kind in ("decode", "prefill", "host"):
         nh, nkv, hd = c["nh"], c["nkv"], c["hd"]
         L, n = c.get("layers", 1), c.get("rows", 1)
