@@ -32,7 +32,7 @@ struct kore_attn {
                                              // the roped q of the generic decode
     int max_split = 0;
     size_t part_floats = 0;
-    bool fast_decode = false, fast_prefill = false;   // MFMA kernels for this geometry
+    bool fast_decode = false;                // MFMA decode kernels for this geometry
     float *d_pf_part = nullptr;              // prefill key-segment partials
     size_t pf_part_floats = 0;
     float *d_scratch = nullptr;              // the device's fixed scratch (allocation-free decode)
@@ -253,24 +253,6 @@ int prefill_enqueue(kore_attn *h, int layer, int pos0, int n_tok, const float *q
     ap.n_tok = n_tok;
     ap.n_head_kv = h->n_head_kv;
     HIP_TRY(h, launch_append(ap, h->head_dim, s));
-    if (!h->fast_prefill) {
-        GenericArgs ga{};
-        ga.q = q;
-        ga.cs = h->d_cs;
-        ga.kc = ap.kc;
-        ga.vc = ap.vc;
-        ga.out = out;
-        ga.slots = h->ctx;
-        ga.hd = h->head_dim;
-        ga.n_head_kv = h->n_head_kv;
-        ga.n_rep = h->n_head / h->n_head_kv;
-        generic_shape(ga.hd, ga.n_rep, &ga.tile, &ga.chunk, &ga.n_chunks);
-        ga.pos0 = pos0;
-        ga.n_split = 1;
-        ga.scale = 1.0f / std::sqrt((float)h->head_dim);   // kore.cpp:1411
-        HIP_TRY(h, launch_generic_prefill(ga, n_tok, s));
-        return KORE_ATTN_OK;
-    }
     PrefillArgs pa{};
     pa.q = q;
     pa.cs = h->d_cs;
@@ -282,32 +264,19 @@ int prefill_enqueue(kore_attn *h, int layer, int pos0, int n_tok, const float *q
     pa.n_tok = n_tok;
     pa.n_head_kv = h->n_head_kv;
     pa.n_rep = h->n_head / h->n_head_kv;
-    pa.n_strips = (n_tok + 31) / 32;
-    pa.scale_log2 = (1.0f / std::sqrt((float)h->head_dim)) * 1.4426950408889634f;
-    pa.n_kseg = prefill_key_segments(n_tok, pos0, h->n_head_kv, pa.n_rep, h->num_cu, &pa.seg_tiles);
-    pa.fold = h->num_cu;
-    if (pa.n_kseg > 1) {
-        const size_t entries = (size_t)h->n_head_kv * pa.n_rep * pa.n_strips * pa.n_kseg * 32;
-        const size_t need = entries * ((size_t)h->head_dim + 2);
-        if (need > h->pf_part_floats)   // cannot happen: sized at create for the largest split
-            return fail(h, KORE_ATTN_E_UNSUPPORTED, "prefill partials need %zu floats, scratch holds %zu", need,
-                        h->pf_part_floats);
+    pa.hd = h->head_dim;
+    pa.scale_log2 = (float)(1.0f / std::sqrt((float)h->head_dim) * 1.4426950408889634);   // kore.cpp:1411
+    prefill_plan(pa, h->num_cu);
+    const size_t ranges = pa.n_split > 0 ? (size_t)pa.n_split * 2 : pa.n_kseg > 1 ? (size_t)pa.n_items * pa.n_kseg : 0;
+    if (ranges) {
+        const size_t rows = (size_t)h->n_head_kv * ranges * kPrefillRows, hdp = (size_t)prefill_padded_dim(h->head_dim);
+        if (rows * (hdp + 2) > h->pf_part_floats)   // cannot happen: sized at create for the largest plan
+            return fail(h, KORE_ATTN_E_UNSUPPORTED, "prefill partials need %zu floats, scratch holds %zu",
+                        rows * (hdp + 2), h->pf_part_floats);
         pa.part_o = h->d_pf_part;
-        pa.part_ml = h->d_pf_part + entries * h->head_dim;
-    } else {
-        prefill_split_plan(pa, h->num_cu);
-        if (pa.n_split > 0) {
-            // n_head_kv * n_split < num_cu items, 4 waves x 2 halves x 32 rows each
-            const size_t entries = (size_t)h->n_head_kv * pa.n_split * 8 * 32;
-            const size_t need = entries * ((size_t)h->head_dim + 2);
-            if (need > h->pf_part_floats)   // cannot happen: sized at create for 8 x num_cu x 32 rows
-                return fail(h, KORE_ATTN_E_UNSUPPORTED, "prefill partials need %zu floats, scratch holds %zu",
-                            need, h->pf_part_floats);
-            pa.part_o = h->d_pf_part;
-            pa.part_ml = h->d_pf_part + entries * h->head_dim;
-        }
+        pa.part_ml = h->d_pf_part + rows * hdp;
     }
-    HIP_TRY(h, launch_prefill(pa, h->head_dim, s));
+    HIP_TRY(h, launch_prefill(pa, s));
     return KORE_ATTN_OK;
 }
 
@@ -369,7 +338,6 @@ int kore_attn_create(kore_attn_t *out, int n_layer, int ctx, int n_head, int n_h
     h->window = window;
     h->rope_base = rope_base;
     h->fast_decode = decode_supported(head_dim, n_rep);
-    h->fast_prefill = prefill_supported(head_dim, n_rep);
     auto bail = [&](hipError_t e, const char *what) {
         g_create_error = std::string(what) + ": " + hipGetErrorString(e);
         release(h);
@@ -406,17 +374,10 @@ int kore_attn_create(kore_attn_t *out, int n_layer, int ctx, int n_head, int n_h
     h->part_floats = np * ((size_t)head_dim + 2) + (h->fast_decode ? 0 : (size_t)n_head * head_dim);
     if ((e = hipMalloc(&h->d_part_o, h->part_floats * sizeof(float))) != hipSuccess)
         return bail(e, "hipMalloc");
-    // Prefill key-segment partials, sized for the largest split any chunk
-    // gets: segments are only used while a chunk has fewer workgroups than
-    // CUs, which bounds (heads x strips x segments) by 8 x num_cu
-    // (prefill_key_segments), i.e. 8 x num_cu x 32 rows of (hd + 2) floats;
-    // a split plan (prefill_split_plan) halves fewer than num_cu items of 4
-    // entries: under 8 x num_cu entries as well.
-    if (h->fast_prefill) {
-        h->pf_part_floats = (size_t)8 * h->num_cu * 32 * ((size_t)head_dim + 2);
-        if ((e = hipMalloc(&h->d_pf_part, h->pf_part_floats * sizeof(float))) != hipSuccess)
-            return bail(e, "hipMalloc");
-    }
+    // Prefill partials of the largest plan: key segments and split halves are
+    // used only where they keep the launch to two workgroups per CU
+    h->pf_part_floats = prefill_part_floats(head_dim, h->num_cu);
+    if ((e = hipMalloc(&h->d_pf_part, h->pf_part_floats * sizeof(float))) != hipSuccess) return bail(e, "hipMalloc");
     // the device's fixed scratch of kore_attn_decode_noalloc_dev, resolved
     // once per device with that device current
     if ((e = static_scratch(h->device, &h->d_scratch)) != hipSuccess) return bail(e, "hipGetSymbolAddress");

@@ -65,7 +65,10 @@ struct AppendArgs {
 };
 
 // Batched causal attention of n_tok query rows at positions pos0.. against
-// cache rows [0, pos0 + n_tok) (kore.cpp:1542-1563).  q is pre-RoPE.
+// cache rows [0, pos0 + n_tok) (kore.cpp:1542-1563).  q is pre-RoPE.  A
+// kv-head's query rows are one list f = position * n_rep + head, cut into
+// items of kPrefillRows (one workgroup each), item 0 the last rows.
+constexpr int kPrefillRows = 128;
 constexpr int kMaxPrefillUnits = 512;   // work units per kv-head of a split plan
 struct PrefillArgs {
     const float *q;       // [n_tok][n_head][hd]
@@ -73,19 +76,20 @@ struct PrefillArgs {
     const float *kc, *vc; // layer base
     float *out;           // [n_tok][n_head][hd]
     int slots;
+    int hd;
     int pos0;
     int n_tok;
     int n_head_kv;
     int n_rep;
-    int n_strips;         // ceil(n_tok / 32)
+    int n_items;          // ceil(n_tok * n_rep / kPrefillRows)
     float scale_log2;     // kore's 1/sqrt(hd) times log2(e)
     // Key segments: with n_kseg > 1 every workgroup item is split into
     // n_kseg launches over key tiles [seg * seg_tiles, (seg + 1) * seg_tiles)
     // that write unnormalised partials, merged by the prefill combine kernel.
     int n_kseg;
     int seg_tiles;
-    float *part_o;        // [n_head_kv * n_rep * n_strips][n_kseg][32][hd]
-    float *part_ml;       // [n_head_kv * n_rep * n_strips][n_kseg][32][2]
+    float *part_o;        // [n_head_kv][n_items][4 strips][n_kseg][32][padded hd]
+    float *part_ml;       // [n_head_kv][n_items][4 strips][n_kseg][32][2]
     // Workgroups b and b + fold (fold = CU count) usually share a CU: the
     // grid index is folded so that the second one runs the work list from
     // its short end (work index grid - 1 - (b - fold) for b >= fold).
@@ -93,7 +97,7 @@ struct PrefillArgs {
     // Split plan (n_kseg == 1, between one and two workgroups per CU): items
     // 0 .. n_split - 1 of every kv-head (the longest) run as two workgroups
     // over the first and second half of their key tiles and write partials
-    // [n_head_kv][n_split][4 waves][2 halves][32] (o, then max / sum), merged
+    // [n_head_kv][n_split][4 strips][2 halves][32] (o, then max / sum), merged
     // by the prefill combine kernel; the other items run whole.  unit[r] is
     // the r-th longest of a kv-head's n_units work units, item << 2 | part
     // (part 0 whole, 1 first half, 2 second half); work index w runs unit
@@ -103,27 +107,30 @@ struct PrefillArgs {
     int n_units;
     uint16_t unit[kMaxPrefillUnits];
 };
+// Fills n_items, the key segments, the fold and the split plan from the
+// chunk's sizes; the partials of any plan take at most prefill_part_floats.
+void prefill_plan(PrefillArgs &a, int num_cu);
+size_t prefill_part_floats(int head_dim, int num_cu);
+int prefill_padded_dim(int head_dim);
+hipError_t launch_prefill(const PrefillArgs &a, hipStream_t s);
 
-// Any even head_dim up to kMaxGenericHeadDim and any n_rep (the geometries
-// kore accepts, kore.cpp:1278-1290, that the MFMA kernels above do not
+// Decode of any even head_dim up to kMaxGenericHeadDim and any n_rep (the
+// geometries kore accepts, kore.cpp:1278-1290, that the MFMA decode does not
 // cover): tiled attention on VALU with fp64 scores.  A workgroup takes `chunk`
-// q-heads of one kv-head and one key range: a decode split of the cache rows
-// (after a prep launch has roped q and appended the new row), or all keys
-// 0..pos of one prefill row.
+// q-heads of one kv-head and one split of the cache rows (after a prep launch
+// has roped q and appended the new row).
 constexpr int kMaxGenericHeadDim = 2 * kMaxRopeHalf;
 constexpr int kMaxGenericSplits = 128;   // decode splits per kv-head of the generic kernels
 struct GenericArgs {
-    const float *q;       // decode: roped q [n_head][hd]; prefill: pre-RoPE q [n_tok][n_head][hd]
-    const float2 *cs;     // prefill: RoPE table (row p = position p); decode: null
+    const float *q;       // roped q [n_head][hd]
     const float *kc, *vc; // layer base
-    float *out;           // [n_tok][n_head][hd]
-    float *part_o;        // decode with n_split > 1: [n_head][n_split][hd]
-    float *part_ml;       //                          [n_head][n_split][2]
+    float *out;           // [n_head][hd]
+    float *part_o;        // with n_split > 1: [n_head][n_split][hd]
+    float *part_ml;       //                   [n_head][n_split][2]
     int slots, hd, n_head_kv, n_rep;
     int chunk, n_chunks;  // q-heads per workgroup, workgroups per kv-head
     int tile;             // keys per LDS tile
-    int pos0;             // prefill: position of row 0
-    int n_rows;           // decode: cache rows attended, [0, n_rows), the new row included
+    int n_rows;           // cache rows attended, [0, n_rows), the new row included
     int rows_per_split, n_split;
     float scale;          // kore's 1/sqrt(hd) (kore.cpp:1411)
 };
@@ -138,8 +145,6 @@ size_t generic_lds_bytes(int head_dim, int tile, int chunk);
 hipError_t launch_generic_decode(const GenericArgs &a, const float *q, const float *k, const float *v,
                                  float *q_out, float *kc, float *vc, int n_head, int new_slot, const RopeRow &rr,
                                  hipStream_t s);
-// Prefill rows after their append: grid (n_tok, n_head_kv * n_chunks).
-hipError_t launch_generic_prefill(const GenericArgs &a, int n_tok, hipStream_t s);
 
 // Counter-based synthetic inputs (identical bits to the CPU oracle's
 // generator): dst[r*dim + c] for r < rows.
@@ -165,19 +170,11 @@ hipError_t static_scratch(int device, float **ptr);
 // Rows per split the decode uses for n_rows cache rows (the host sizes the
 // partial buffers from the maximum split count over all lengths).
 int decode_rows_per_split(int head_dim, int n_rows, int n_head_kv, int num_cu);
-// Geometries of the MFMA decode / prefill kernels; the others take the
-// generic kernels.
+// Geometries of the MFMA decode kernels; the others take the generic ones.
 bool decode_supported(int head_dim, int n_rep);
-bool prefill_supported(int head_dim, int n_rep);
 
 hipError_t launch_decode(const DecodeArgs &a, const RopeRow &rr, int head_dim, hipStream_t s);
 hipError_t launch_append(const AppendArgs &a, int head_dim, hipStream_t s);
-hipError_t launch_prefill(const PrefillArgs &a, int head_dim, hipStream_t s);
-// Key segments the prefill uses for n_tok rows at pos0 (1 = none).
-int prefill_key_segments(int n_tok, int pos0, int n_head_kv, int n_rep, int num_cu, int *seg_tiles);
-// Fills a.n_split / a.n_units / a.unit for a chunk without key segments (its
-// other fields set); n_split stays 0 where the plan does not apply.
-void prefill_split_plan(PrefillArgs &a, int num_cu);
 hipError_t launch_synth(const SynthArgs &a, hipStream_t s);
 
 }  // namespace kore_attn_gpu

@@ -16,15 +16,11 @@
 //                          workgroup and one workgroup reading every partial
 //                          serialises the merge.
 //   append_kernel   RoPE + append of a prefill chunk (kore.cpp:1535-1538).
-//   prefill_kernel  causal attention of a prefill chunk (kore.cpp:1542-1563)
-//                   on fp32 MFMA (v_mfma_f32_32x32x2_f32) with LDS-staged K and
-//                   transposed V tiles shared by the four waves of a
-//                   workgroup, which all belong to one kv-head (GQA sharing).
-//   generic_*       every other geometry kore accepts (any even head_dim up
-//                   to 256, any q-heads per kv-head): a decode prep launch
+//   generic_*       decode of every other geometry kore accepts (any even
+//                   head_dim up to 256, any q-heads per kv-head): a prep launch
 //                   (RoPE of q, RoPE + append of the new row), LDS-tiled
-//                   attention on VALU with fp64 scores for decode splits and
-//                   prefill rows, and the merge of the decode's split partials.
+//                   attention on VALU with fp64 scores for the splits, and the
+//                   merge of their partials.
 //   synth_kernel    counter-based synthetic inputs for benchmarks and tests.
 //
 // RoPE is bit-exact with kore: cos/sin come from the host-built table (the
@@ -34,6 +30,7 @@
 // built with -ffp-contract=off; fused multiply-adds below are explicit
 // fmaf() calls or MFMA instructions.
 #include "kore_attn_kernels.h"
+#include "kore_attn_device.h"
 
 #include <algorithm>
 #include <cmath>
@@ -43,36 +40,7 @@
 namespace kore_attn_gpu {
 namespace {
 
-constexpr int kThreads = 256;
-constexpr int kWaves = 4;
 constexpr size_t kLdsPerCu = 160 * 1024;   // gfx950
-
-typedef float floatx16 __attribute__((ext_vector_type(16)));
-typedef float floatx4 __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ float4 ld4(const float *p) { return *reinterpret_cast<const float4 *>(p); }
-__device__ __forceinline__ void st4(float *p, float4 v) { *reinterpret_cast<float4 *>(p) = v; }
-__device__ __forceinline__ float4 zero4() { return make_float4(0.f, 0.f, 0.f, 0.f); }
-__device__ __forceinline__ float comp(const float4 &v, int e) {
-    return e == 0 ? v.x : (e == 1 ? v.y : (e == 2 ? v.z : v.w));
-}
-
-
-// Cross-lane moves inside a 16-lane DPP row (no LDS traffic).  CTRL is a
-// DPP control word: 0x121..0x12F rotate the row right by 1..15 lanes,
-// 0x141 mirrors each half-row of 8 lanes, 0x00..0xFF permute within quads.
-template <int CTRL>
-__device__ __forceinline__ float dpp(float x) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xF, 0xF, false));
-}
-// Max over each 16-lane row; every lane of the row receives it.
-__device__ __forceinline__ float row16_max(float x) {
-    x = fmaxf(x, dpp<0x128>(x));
-    x = fmaxf(x, dpp<0x124>(x));
-    x = fmaxf(x, dpp<0x122>(x));
-    return fmaxf(x, dpp<0x121>(x));
-}
-__device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
 // Timing build only (libkore_attn_tl.so, compiled with -DKORE_DECODE_TIMELINE;
 // never the product library): every wave of the latest decode_split_kernel
@@ -106,16 +74,6 @@ __device__ unsigned long long g_tl_comb[kTlComb * kTlCombStamps];
 #define TL_WRITE(buf, cap, id, n) ((void)0)
 #endif
 
-// NEOX rotation of the pair (x0, x1) = (x[i], x[i + hd/2]) by (c, s)
-// (kore.cpp:1379-1382): products rounded, then difference / sum rounded.
-__device__ __forceinline__ void rope_pair(float x0, float x1, float2 cs, float &y0, float &y1) {
-#pragma clang fp contract(off)
-    const float a = x0 * cs.x, b = x1 * cs.y;
-    const float c = x0 * cs.y, d = x1 * cs.x;
-    y0 = a - b;
-    y1 = c + d;
-}
-
 // ------------------------------------------------------------------ decode
 
 // v_mfma_f32_16x16x4f32, one block: lane l supplies A[l%16][l/16] and
@@ -124,26 +82,6 @@ __device__ __forceinline__ floatx4 mfma16(float a, float b, floatx4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
-// x of lane l and of lane l ^ 16 (v_permlane16_swap with x as both operands
-// returns the even 16-lane rows in one result and the odd rows in the other),
-// and likewise of lane l ^ 32 (v_permlane32_swap).  The results are copied
-// to integers before the bit casts: a bit cast applied to an element of the
-// returned vector directly is compiled as the first element by this hipcc
-// (ROCm 7.2) for either index.
-__device__ __forceinline__ void pair16(float x, float &a, float &b) {
-    const unsigned xb = __builtin_bit_cast(unsigned, x);
-    const auto r = __builtin_amdgcn_permlane16_swap(xb, xb, false, false);
-    const unsigned r0 = r[0], r1 = r[1];
-    a = __builtin_bit_cast(float, r0);
-    b = __builtin_bit_cast(float, r1);
-}
-__device__ __forceinline__ void pair32(float x, float &a, float &b) {
-    const unsigned xb = __builtin_bit_cast(unsigned, x);
-    const auto r = __builtin_amdgcn_permlane32_swap(xb, xb, false, false);
-    const unsigned r0 = r[0], r1 = r[1];
-    a = __builtin_bit_cast(float, r0);
-    b = __builtin_bit_cast(float, r1);
-}
 // Max / sum over the four lanes l % 16 + 16 k (k = 0..3); every one of them
 // receives the same value (the operands are the same in all four lanes).
 __device__ __forceinline__ float max4rows(float x) {
@@ -1206,20 +1144,17 @@ __device__ __forceinline__ float wave_sum(float x) {
 // fp64), times kore's 1/sqrt(hd) and log2(e); one wave per head takes the
 // tile's max and the weights 2^(score - max) with the difference in fp64;
 // then every thread advances its outputs (head, dim) by the weighted V rows
-// in fp32.  Prefill workgroups take row z = blockIdx.x with keys 0..pos0+z
-// and rope their q rows from the table; decode workgroups take split
-// blockIdx.x of the rows [0, n_rows) with q already roped.
+// in fp32.  Workgroups take split blockIdx.x of the rows [0, n_rows) with q
+// already roped.
 __global__ __launch_bounds__(kThreads) void generic_attend_kernel(GenericArgs a) {
     extern __shared__ __align__(16) unsigned char g_lds[];
     const int hd = a.hd, T = a.tile, CH = a.chunk, tid = threadIdx.x;
     const int lane = tid & 63, wave = tid >> 6;
     const int g = blockIdx.y / a.n_chunks, c = blockIdx.y % a.n_chunks;
     const int h0 = c * CH, nh = min(CH, a.n_rep - h0);
-    const int n_head = a.n_head_kv * a.n_rep, hq0 = g * a.n_rep + h0;
-    const bool prefill = a.cs != nullptr;
-    const int z = prefill ? (int)blockIdx.x : 0;
-    const int r_begin = prefill ? 0 : (int)blockIdx.x * a.rows_per_split;
-    const int r_end = prefill ? a.pos0 + z + 1 : min(r_begin + a.rows_per_split, a.n_rows);
+    const int hq0 = g * a.n_rep + h0;
+    const int r_begin = (int)blockIdx.x * a.rows_per_split;
+    const int r_end = min(r_begin + a.rows_per_split, a.n_rows);
 
     double *s_sc = reinterpret_cast<double *>(g_lds);   // [CH][T] scores
     float *s_p = reinterpret_cast<float *>(s_sc + CH * T);   // [CH][T] weights
@@ -1229,18 +1164,8 @@ __global__ __launch_bounds__(kThreads) void generic_attend_kernel(GenericArgs a)
     float *s_k = s_q + CH * hd;                              // [T][hd + 1]
     float *s_v = s_k + T * (hd + 1);                         // [T][hd]
 
-    const float *qb = a.q + ((size_t)z * n_head + hq0) * hd;
-    for (int e = tid; e < nh * hd; e += kThreads) {
-        if (prefill) {
-            const int i = e / hd, d = e % hd, half = hd / 2, d0 = d < half ? d : d - half;
-            const float *qr = qb + (size_t)i * hd;
-            float y0, y1;
-            rope_pair(qr[d0], qr[d0 + half], a.cs[(size_t)(a.pos0 + z) * half + d0], y0, y1);
-            s_q[e] = d < half ? y0 : y1;
-        } else {
-            s_q[e] = qb[e];
-        }
-    }
+    const float *qb = a.q + (size_t)hq0 * hd;
+    for (int e = tid; e < nh * hd; e += kThreads) s_q[e] = qb[e];
     if (tid < nh) {
         s_m[tid] = -INFINITY;
         s_l[tid] = 0.f;
@@ -1303,11 +1228,11 @@ __global__ __launch_bounds__(kThreads) void generic_attend_kernel(GenericArgs a)
         }
     }
     __syncthreads();
-    if (prefill || a.n_split == 1) {
+    if (a.n_split == 1) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const int o = tid + j * kThreads;
-            if (o < nh * hd) a.out[((size_t)z * n_head + hq0) * hd + o] = acc[j] / s_l[o / hd];
+            if (o < nh * hd) a.out[(size_t)hq0 * hd + o] = acc[j] / s_l[o / hd];
         }
     } else {
         const int sp = blockIdx.x;
@@ -1342,346 +1267,6 @@ __global__ void generic_combine_kernel(const float *part_o, const float *part_ml
         }
         out[(size_t)h * hd + d] = acc / den;
     }
-}
-
-// ----------------------------------------------------------------- prefill
-
-// v_mfma_f32_32x32x2_f32, one block: lane l supplies A[l%32][l/32] and
-// B[l/32][l%32]; D register r of lane l is D[8(r/4) + 4(l/32) + r%4][l%32].
-__device__ __forceinline__ floatx16 mfma32(float a, float b, floatx16 c) {
-    return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
-}
-
-// Workgroup = 4 waves of one kv-head g; wave w takes entry 4*item + w of g's
-// list of (strip, q-head) pairs ordered by strip descending, so the waves of
-// a workgroup attend the same key range (to within one tile) and share each
-// K / V tile from LDS.  A strip is 32 query rows.  Per 32-key tile a wave
-// computes S^T = K Q^T (keys x queries, 64 MFMAs for hd 128) so that every
-// lane owns the scores of one query, runs the online softmax in base 2 on
-// them, and accumulates O^T += V^T P^T (64 MFMAs), whose D layout again gives
-// each lane one query; the softmax statistics need one cross-lane exchange.
-// The tiles go from HBM straight into LDS (global_load_lds_dwordx4: lane i of
-// a load writes 16 bytes at the wave's base + 16 i), double-buffered, so tile
-// t + 1 streams in while tile t is computed, with one barrier per tile and no
-// staging registers.  V is kept row-major: output block tt of a wave holds
-// dims NT i + tt (i < 32), so one 16-byte (hd 64: 8-byte) read of a V row
-// feeds all NT blocks; K's float4 columns are XOR-swizzled by (row mod 16)
-// so the 16-byte reads of 16 rows at one column fall in different banks.
-// With key segments (a short chunk over a long cache has too few workgroups
-// to fill the GPU) a workgroup covers one range of key tiles and writes its
-// rows' unnormalised output with their max and sum instead.  The strips'
-// causal work runs from 1 to n_tok / 32 tiles; two workgroups share a CU, and
-// the grid is folded (PrefillArgs::fold) to pair long strips with short ones.
-template <int HD>
-__global__ __launch_bounds__(kThreads, 2) void prefill_kernel(PrefillArgs a) {
-    constexpr int BK = 32;
-    constexpr int NT = HD / 32;
-    constexpr int HALF = HD / 2;
-    constexpr int C4 = HD / 4;                 // float4 per cache row
-    constexpr int NI = BK * C4 / 64 / kWaves;  // LDS loads per wave per tensor and tile
-    static_assert(NI * 64 * kWaves == BK * C4, "whole 1 KB loads per tile");
-    // one array per buffer: the compiler tracks LDS-direct loads per LDS
-    // object, so reads of one buffer do not wait for loads into the other
-    __shared__ __align__(16) float sK0[BK * HD], sK1[BK * HD];
-    __shared__ __align__(16) float sV0[BK * HD], sV1[BK * HD];
-
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int nkv = a.n_head_kv;
-    // work index: items run from the longest strips down; the second part
-    // of the grid takes them from the short end, so that the two
-    // workgroups of a CU (b and b + fold) add up to about the same work
-    const int bx = blockIdx.x;
-    const int wi = bx < a.fold ? bx : (int)gridDim.x - 1 - (bx - a.fold);
-    const int g = wi % nkv;
-    // split plan: unit = item << 2 | part (0 whole, 1 / 2 first / second half)
-    const int unit = a.n_split > 0 ? (int)a.unit[wi / nkv] : 0;
-    const int part = unit & 3;
-    const int seg = a.n_split > 0 ? 0 : (wi / nkv) % a.n_kseg;
-    const int item = a.n_split > 0 ? unit >> 2 : wi / nkv / a.n_kseg;
-    const int total = a.n_rep * a.n_strips;
-    const int e = item * 4 + wave;
-    const bool active = e < total;
-    const int ee = active ? e : total - 1;
-    const int strip = a.n_strips - 1 - ee / a.n_rep;
-    const int h = g * a.n_rep + ee % a.n_rep;
-    const int strip0 = a.n_strips - 1 - (item * 4) / a.n_rep;
-    const int n_keys = a.pos0 + a.n_tok;
-    const int wg_kmax = min(a.pos0 + 32 * strip0 + 31, n_keys - 1);
-    const int my_kmax = active ? min(a.pos0 + 32 * strip + 31, n_keys - 1) : -1;
-    const int n_tiles = wg_kmax / BK + 1;
-    const int n_head = nkv * a.n_rep;
-
-    const int qi = lane & 31, qg = lane >> 5;
-    const int qrow = 32 * strip + qi;
-    const bool qvalid = active && qrow < a.n_tok;
-    const int qrow_c = min(qrow, a.n_tok - 1);
-    const int qpos = a.pos0 + qrow_c;
-
-    // Q^T operand: qreg[4j+e] = roped q[qrow][8j + 4qg + e] * 1/sqrt(hd) * log2(e),
-    // filled after the first key tile is requested (its loads then overlap q's)
-    float qreg[HD / 2];
-    auto load_q = [&] {
-        const float *qp = a.q + ((size_t)qrow_c * n_head + h) * HD;
-        const float2 *cs = a.cs + (size_t)qpos * HALF;
-#pragma unroll
-        for (int j = 0; j < HD / 16; ++j) {
-            const int d = 8 * j + 4 * qg;
-            const float4 lo = qvalid ? ld4(qp + d) : zero4();
-            const float4 hi = qvalid ? ld4(qp + HALF + d) : zero4();
-#pragma unroll
-            for (int e2 = 0; e2 < 4; ++e2) {
-                float y0, y1;
-                rope_pair(comp(lo, e2), comp(hi, e2), cs[d + e2], y0, y1);
-                qreg[4 * j + e2] = y0 * a.scale_log2;
-                qreg[4 * (j + HD / 16) + e2] = y1 * a.scale_log2;
-            }
-        }
-    };
-
-    floatx16 acc[NT];
-#pragma unroll
-    for (int t = 0; t < NT; ++t)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[t][r] = 0.f;
-    float m_run = -INFINITY, l_run = 0.f;
-
-    // Tile t into (dK, dV): load i of wave w covers float4 slots
-    // p = 64 (NI w + i) + lane, i.e. row p / C4 and position p % C4; V holds
-    // column (p % C4) there, K column (p % C4) ^ (row & 15).  Keys past the
-    // cache end are clamped to its last row (the causal mask excludes them:
-    // every query position is below n_keys).
-    const int wave_u = __builtin_amdgcn_readfirstlane(wave);
-    auto issue_tile = [&](float *dK, float *dV, int t) {
-        if (t * BK + BK <= n_keys) {
-            const size_t tb = ((size_t)g * a.slots + t * BK) * HD;
-            const float *kb = a.kc + tb, *vb = a.vc + tb;
-#pragma unroll
-            for (int i = 0; i < NI; ++i) {
-                // per-lane offsets inside a tile, the same for every tile
-                const int chunk = NI * wave_u + i;
-                const int p = 64 * chunk + lane;
-                const int row = p / C4, pos = p % C4;
-                const int koff = row * HD + 4 * (pos ^ (row & 15)), voff = row * HD + 4 * pos;
-                __builtin_amdgcn_global_load_lds(kb + koff, (void __attribute__((address_space(3))) *)(dK + 256 * chunk), 16, 0, 0);
-                __builtin_amdgcn_global_load_lds(vb + voff, (void __attribute__((address_space(3))) *)(dV + 256 * chunk), 16, 0, 0);
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < NI; ++i) {
-                const int chunk = NI * wave_u + i;
-                const int p = 64 * chunk + lane;
-                const int row = p / C4, pos = p % C4;
-                const size_t base = ((size_t)g * a.slots + min(t * BK + row, n_keys - 1)) * HD;
-                __builtin_amdgcn_global_load_lds(a.kc + base + 4 * (pos ^ (row & 15)),
-                                                 (void __attribute__((address_space(3))) *)(dK + 256 * chunk), 16, 0, 0);
-                __builtin_amdgcn_global_load_lds(a.vc + base + 4 * pos,
-                                                 (void __attribute__((address_space(3))) *)(dV + 256 * chunk), 16, 0, 0);
-            }
-        }
-    };
-    auto compute_tile = [&](const float *sK, const float *sV, int t) {
-        const int k0 = t * BK;
-        if (k0 > my_kmax) return;
-        floatx16 s;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) s[r] = 0.f;
-#pragma unroll
-        for (int j = 0; j < HD / 8; ++j) {
-            const float4 a4 = ld4(&sK[qi * HD + 4 * ((2 * j + qg) ^ (qi & 15))]);
-            s = mfma32(a4.x, qreg[4 * j + 0], s);
-            s = mfma32(a4.y, qreg[4 * j + 1], s);
-            s = mfma32(a4.z, qreg[4 * j + 2], s);
-            s = mfma32(a4.w, qreg[4 * j + 3], s);
-        }
-        // s[r] = score(query qi, key k0 + 8(r/4) + 4qg + r%4), already in the
-        // log2 domain; the causal mask only matters on tiles that reach past
-        // the strip's first query position
-        if (k0 + BK - 1 > a.pos0 + 32 * strip) {
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int key = k0 + 8 * (r / 4) + 4 * qg + (r % 4);
-                if (key > qpos) s[r] = -INFINITY;
-            }
-        }
-        float mt = s[0];
-#pragma unroll
-        for (int r = 1; r < 16; ++r) mt = fmaxf(mt, s[r]);
-        {
-            float lo, hi;
-            pair32(mt, lo, hi);
-            mt = fmaxf(lo, hi);
-        }
-        // Each query keeps a reference maximum and moves it only when the new
-        // maximum exceeds it by more than 8 (log2 units): the exponentials
-        // stay below 2^8 and the accumulator rescale is skipped for most
-        // tiles (any reference gives the same normalised result).
-        const float m_max = fmaxf(m_run, mt);
-        const float m_new = (m_max > m_run + 8.f || m_run == -INFINITY) ? m_max : m_run;
-        // a segment may start with a tile that is all masked for a row
-        const float m_use = m_new == -INFINITY ? 0.f : m_new;
-        const float alpha = fast_exp2(m_run - m_use);
-        float psum = 0.f;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            s[r] = fast_exp2(s[r] - m_use);
-            psum += s[r];
-        }
-        {
-            float lo, hi;
-            pair32(psum, lo, hi);
-            psum = lo + hi;
-        }
-        l_run = fmaf(l_run, alpha, psum);
-        m_run = m_new;
-        // rescale only when some query's running max moved
-        if (__builtin_amdgcn_ballot_w64(alpha != 1.f)) {
-#pragma unroll
-            for (int tt = 0; tt < NT; ++tt)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) acc[tt][r] *= alpha;
-        }
-        // PV: k-step (sb, e) takes key 8sb + 4qg + e of the tile
-#pragma unroll
-        for (int sb = 0; sb < 4; ++sb)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const float *vr = &sV[(8 * sb + 4 * qg + e) * HD + NT * qi];
-                if constexpr (NT == 4) {
-                    const float4 v4 = ld4(vr);
-                    acc[0] = mfma32(v4.x, s[4 * sb + e], acc[0]);
-                    acc[1] = mfma32(v4.y, s[4 * sb + e], acc[1]);
-                    acc[2] = mfma32(v4.z, s[4 * sb + e], acc[2]);
-                    acc[3] = mfma32(v4.w, s[4 * sb + e], acc[3]);
-                } else {
-                    const float2 v2 = *reinterpret_cast<const float2 *>(vr);
-                    acc[0] = mfma32(v2.x, s[4 * sb + e], acc[0]);
-                    acc[1] = mfma32(v2.y, s[4 * sb + e], acc[1]);
-                }
-            }
-    };
-
-    // key tiles of this workgroup: a key segment, a half of a split item
-    // (the plan splits only items of at least two tiles), or all of them
-    const int t_half = n_tiles / 2;
-    const int t_begin = part == 2 ? t_half : seg * a.seg_tiles;
-    const int t_end = part == 1 ? t_half : (a.n_kseg == 1 ? n_tiles : min(n_tiles, t_begin + a.seg_tiles));
-    if (t_begin < t_end) issue_tile(sK0, sV0, t_begin);
-    load_q();
-    for (int t = t_begin; t < t_end; t += 2) {
-        // this wave's loads of tile t have landed; after the barrier every
-        // wave's have, and every wave is done with the other buffer
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
-        if (t + 1 < t_end) issue_tile(sK1, sV1, t + 1);
-        compute_tile(sK0, sV0, t);
-        if (t + 1 >= t_end) break;
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
-        if (t + 2 < t_end) issue_tile(sK0, sV0, t + 2);
-        compute_tile(sK1, sV1, t + 1);
-    }
-
-    // output: lane (qi, qg) register r of block tt is dim NT i + tt with
-    // i = 8 (r / 4) + 4 qg + r % 4, so the NT blocks give NT consecutive dims
-    auto store_row = [&](float *dst, float sc) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int i = 8 * (r / 4) + 4 * qg + (r % 4);
-            if constexpr (NT == 4)
-                st4(dst + 4 * i, make_float4(acc[0][r] * sc, acc[1][r] * sc, acc[2][r] * sc, acc[3][r] * sc));
-            else
-                *reinterpret_cast<float2 *>(dst + 2 * i) = make_float2(acc[0][r] * sc, acc[1][r] * sc);
-        }
-    };
-    if (a.n_kseg > 1 || part != 0) {
-        if (!active) return;
-        const size_t pe = part != 0 ? (((size_t)g * a.n_split + item) * 4 + wave) * 2 + (part - 1)
-                                    : ((size_t)g * total + ee) * a.n_kseg + seg;
-        store_row(a.part_o + (pe * 32 + qi) * HD, 1.f);
-        if (qg == 0) {
-            a.part_ml[(pe * 32 + qi) * 2 + 0] = m_run;
-            a.part_ml[(pe * 32 + qi) * 2 + 1] = l_run;
-        }
-        return;
-    }
-    if (qvalid) store_row(a.out + ((size_t)qrow * n_head + h) * HD, 1.f / l_run);
-}
-
-// Block = one (kv-head, strip, q-head) entry of the prefill: the log-sum-exp
-// merge of its key segments (or of the two halves of a split item) for 32
-// query rows; thread (row r, chunk c) owns HD / 8 dims of one row.
-template <int HD>
-__global__ __launch_bounds__(256) void prefill_combine_kernel(PrefillArgs a) {
-    constexpr int CH = HD / 8;                          // dims per thread
-    const int total = a.n_rep * a.n_strips;
-    int g, e, S;
-    size_t base;
-    if (a.n_split > 0) {
-        // block = (kv-head, split item, wave) of the split plan
-        const int id = blockIdx.x, gi = id >> 2;
-        g = gi / a.n_split;
-        e = (gi - g * a.n_split) * 4 + (id & 3);
-        if (e >= total) return;
-        S = 2;
-        base = (size_t)id * 2;
-    } else {
-        const int entry = blockIdx.x;
-        g = entry / total;
-        e = entry - g * total;
-        S = a.n_kseg;
-        base = (size_t)entry * S;
-    }
-    const int strip = a.n_strips - 1 - e / a.n_rep;
-    const int h = g * a.n_rep + e % a.n_rep;
-    const int r = threadIdx.x >> 3, c = threadIdx.x & 7;
-    const int qrow = 32 * strip + r;
-    if (qrow >= a.n_tok) return;
-    // segments in batches of four, every load of a batch issued before its
-    // arithmetic (one memory round trip per batch); the sums in segment order
-    constexpr int kSeg = 4;
-    const float2 *ml = reinterpret_cast<const float2 *>(a.part_ml);
-    float m = -INFINITY;
-    for (int s0 = 0; s0 < S; s0 += 2 * kSeg) {
-        float mv[2 * kSeg];
-#pragma unroll
-        for (int u = 0; u < 2 * kSeg; ++u) mv[u] = s0 + u < S ? ml[(base + s0 + u) * 32 + r].x : -INFINITY;
-#pragma unroll
-        for (int u = 0; u < 2 * kSeg; ++u) m = fmaxf(m, mv[u]);
-    }
-    float den = 0.f;
-    float4 acc[CH / 4];
-#pragma unroll
-    for (int j = 0; j < CH / 4; ++j) acc[j] = zero4();
-    for (int s0 = 0; s0 < S; s0 += kSeg) {
-        float2 st[kSeg];
-        float4 x[kSeg][CH / 4];
-#pragma unroll
-        for (int u = 0; u < kSeg; ++u)
-            if (s0 + u < S) {
-                st[u] = ml[(base + s0 + u) * 32 + r];
-                const float *po = a.part_o + ((base + s0 + u) * 32 + r) * HD + c * CH;
-#pragma unroll
-                for (int j = 0; j < CH / 4; ++j) x[u][j] = ld4(po + 4 * j);
-            }
-#pragma unroll
-        for (int u = 0; u < kSeg; ++u)
-            if (s0 + u < S) {
-                const float w = st[u].x == -INFINITY ? 0.f : exp2f(st[u].x - m);
-                den = fmaf(w, st[u].y, den);
-#pragma unroll
-                for (int j = 0; j < CH / 4; ++j) {
-                    acc[j].x = fmaf(w, x[u][j].x, acc[j].x);
-                    acc[j].y = fmaf(w, x[u][j].y, acc[j].y);
-                    acc[j].z = fmaf(w, x[u][j].z, acc[j].z);
-                    acc[j].w = fmaf(w, x[u][j].w, acc[j].w);
-                }
-            }
-    }
-    const float inv = 1.f / den;
-    float *op = a.out + ((size_t)qrow * a.n_head_kv * a.n_rep + h) * HD + c * CH;
-#pragma unroll
-    for (int j = 0; j < CH / 4; ++j)
-        st4(op + 4 * j, make_float4(acc[j].x * inv, acc[j].y * inv, acc[j].z * inv, acc[j].w * inv));
 }
 
 // ------------------------------------------------------------------- synth
@@ -1833,10 +1418,6 @@ bool decode_supported(int head_dim, int n_rep) {
     return (head_dim == 64 || head_dim == 128) && n_rep >= 1 && n_rep <= 8;
 }
 
-bool prefill_supported(int head_dim, int n_rep) {
-    return (head_dim == 64 || head_dim == 128) && n_rep >= 1;
-}
-
 int decode_rows_per_split(int head_dim, int n_rows, int n_head_kv, int num_cu) {
     // S = num_cu / n_head_kv splits per kv-head (one workgroup per CU; at
     // most kMaxDecodeSplits, and at least kDecodeBlock rows per split) of
@@ -1890,77 +1471,6 @@ hipError_t launch_append(const AppendArgs &a, int head_dim, hipStream_t s) {
     return hipGetLastError();
 }
 
-int prefill_key_segments(int n_tok, int pos0, int n_head_kv, int n_rep, int num_cu, int *seg_tiles) {
-    // Split the key range when the workgroups of a chunk do not fill every
-    // CU (two fit per CU): as many segments as keep all of them in one wave
-    // of two per CU, each of at least 2 key tiles.  A 64-row chunk has 16
-    // workgroups (7B): unsplit, each walks all its key tiles alone.
-    const int n_strips = (n_tok + 31) / 32;
-    const int n_wg = (n_rep * n_strips + 3) / 4 * n_head_kv;
-    const int n_tiles = (pos0 + n_tok - 1) / 32 + 1;
-    int n_kseg = 1;
-    if (n_wg < num_cu)
-        n_kseg = std::max(1, std::min(2 * num_cu / n_wg, n_tiles / 2));
-    *seg_tiles = (n_tiles + n_kseg - 1) / n_kseg;
-    return n_kseg;
-}
-
-void prefill_split_plan(PrefillArgs &a, int num_cu) {
-    // Two workgroups fit per CU and the grid is folded so that each CU's pair
-    // adds up to about the mean work; with between one and two workgroups per
-    // CU some CUs hold one item only, while the pairs' sums run up to about
-    // the longest item plus the shortest.  Splitting the longest items into
-    // two halves of their key tiles fills the grid to two per CU and lets the
-    // pairs (r-th longest unit with the r-th shortest) even out.
-    a.n_split = 0;
-    a.n_units = 0;
-    const int items = (a.n_rep * a.n_strips + 3) / 4;
-    const int n_wg = items * a.n_head_kv;
-    if (a.n_kseg != 1 || n_wg < num_cu || n_wg >= 2 * num_cu) return;
-    const int n_keys = a.pos0 + a.n_tok;
-    auto tiles = [&](int i) {   // key tiles of item i (its first entry's strip)
-        const int strip0 = a.n_strips - 1 - (4 * i) / a.n_rep;
-        return std::min(a.pos0 + 32 * strip0 + 31, n_keys - 1) / 32 + 1;
-    };
-    int split = std::min(items, (2 * num_cu - n_wg) / a.n_head_kv);
-    while (split > 0 && tiles(split - 1) < 4) --split;   // halves of at least two tiles
-    if (split == 0 || items + split > kMaxPrefillUnits) return;
-    struct Unit { int tiles, code; };
-    std::vector<Unit> u;
-    u.reserve(items + split);
-    for (int i = 0; i < items; ++i) {
-        const int t = tiles(i);
-        if (i < split) {
-            u.push_back({t / 2, i << 2 | 1});
-            u.push_back({t - t / 2, i << 2 | 2});
-        } else {
-            u.push_back({t, i << 2});
-        }
-    }
-    std::stable_sort(u.begin(), u.end(), [](const Unit &x, const Unit &y) { return x.tiles > y.tiles; });
-    for (size_t r = 0; r < u.size(); ++r) a.unit[r] = (uint16_t)u[r].code;
-    a.n_split = split;
-    a.n_units = (int)u.size();
-}
-
-hipError_t launch_prefill(const PrefillArgs &a, int head_dim, hipStream_t s) {
-    const int items = (a.n_rep * a.n_strips + 3) / 4;
-    const dim3 grid(a.n_split > 0 ? a.n_units * a.n_head_kv : items * a.n_head_kv * a.n_kseg);
-    if (head_dim == 128) hipLaunchKernelGGL(prefill_kernel<128>, grid, dim3(kThreads), 0, s, a);
-    else if (head_dim == 64) hipLaunchKernelGGL(prefill_kernel<64>, grid, dim3(kThreads), 0, s, a);
-    else return hipErrorInvalidValue;
-    if (a.n_split > 0) {
-        const dim3 cgrid(a.n_head_kv * a.n_split * 4);
-        if (head_dim == 128) hipLaunchKernelGGL(prefill_combine_kernel<128>, cgrid, dim3(256), 0, s, a);
-        else hipLaunchKernelGGL(prefill_combine_kernel<64>, cgrid, dim3(256), 0, s, a);
-    } else if (a.n_kseg > 1) {
-        const dim3 cgrid(a.n_head_kv * a.n_rep * a.n_strips);
-        if (head_dim == 128) hipLaunchKernelGGL(prefill_combine_kernel<128>, cgrid, dim3(256), 0, s, a);
-        else hipLaunchKernelGGL(prefill_combine_kernel<64>, cgrid, dim3(256), 0, s, a);
-    }
-    return hipGetLastError();
-}
-
 bool generic_supported(int head_dim) {
     return head_dim >= 2 && head_dim <= kMaxGenericHeadDim && head_dim % 2 == 0;
 }
@@ -2006,12 +1516,6 @@ hipError_t launch_generic_decode(const GenericArgs &a, const float *q, const flo
     if (a.n_split > 1)
         hipLaunchKernelGGL(generic_combine_kernel, dim3(n_head), dim3(std::min(256, (a.hd + 63) / 64 * 64)), 0, s,
                            a.part_o, a.part_ml, a.out, a.n_split, a.hd);
-    return hipGetLastError();
-}
-
-hipError_t launch_generic_prefill(const GenericArgs &a, int n_tok, hipStream_t s) {
-    const size_t lds = generic_lds_bytes(a.hd, a.tile, a.chunk);
-    hipLaunchKernelGGL(generic_attend_kernel, dim3(n_tok, a.n_head_kv * a.n_chunks), dim3(kThreads), lds, s, a);
     return hipGetLastError();
 }
 

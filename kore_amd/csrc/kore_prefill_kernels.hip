@@ -1,0 +1,799 @@
+// kore_prefill_kernels.hip - gfx950 kernels of kore's batched causal attention
+// (forward_batch(), kore.cpp:1542-1563), any even head_dim up to 256 and any
+// number of q-heads per kv-head.
+//
+//   prefill_kernel          causal attention of a chunk of query rows over the
+//                           cache, both products on fp16 MFMA with every
+//                           operand split into two fp16 parts
+//   prefill_combine_kernel  merge of the key ranges that a query row's work
+//                           was split into
+//
+// Why split fp16.  The fp32 matrix rate (157 TFLOP/s) bounds the two products;
+// fp16 runs 16 times as fast, and x = hi + lo with hi = fp16(x), lo = fp16(x -
+// hi) carries 22 bits, so three products (hi hi + hi lo + lo hi, each exact,
+// summed in fp32) cost 3 / 16 of the fp32 ones.  The sums take 16 products per
+// fp32 rounding instead of two, and the score's small cross terms are summed
+// first, so the result is nearer to the exact one than the fp32 kernel's was
+// (28/4/128, 2048 rows: 3.9e-7 of the 2-norm against 7.2e-7).  A head_dim that
+// is neither 64 nor 128 ran on VALU with fp64 scores; to lose nothing there its
+// scores take the fourth product and sum their 16-dim pieces in fp64 (33/3/96,
+// 700 rows: 3.6e-7 both; 4/4/140: 2.0e-7 against 1.8e-7 and 2.1e-7).
+//
+// Measured, one layer, against the kernels before (fp32 MFMA; VALU for 33/3/96):
+// 28/4/128 2048 rows 261 -> 141 us (114 -> 213 TFLOP/s), 12/2/128 333 rows at
+// 7001 151 -> 73 us, 33/3/96 700 rows at 100 731 -> 54 us.  What bounds it now:
+// the MFMAs (39 % of the cycles) and the softmax and split arithmetic (47 %)
+// hardly overlap, since a wave does one after the other.
+//
+// Range.  fp16 holds 2^-24 .. 65504, so every operand is scaled by a power of
+// two (exact) that brings its largest magnitude to 2^13 .. 2^14: a query row
+// by its own, K and V by groups of eight keys, the softmax weights by a fixed
+// one.  What is lost of a small value is then at most 2^-39 of its group's
+// largest.  Infinities and NaN in K or V are handled apart (the `bad` groups),
+// so they reach exactly the rows that an fp32 product would give them to.
+#include "kore_attn_kernels.h"
+#include "kore_attn_device.h"
+
+#include <algorithm>
+#include <vector>
+
+namespace kore_attn_gpu {
+namespace {
+
+typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+typedef float float2v __attribute__((ext_vector_type(2)));
+typedef float float8v __attribute__((ext_vector_type(8)));
+// vectors of floats at any float's address (q, out and odd geometries' rows)
+typedef float f2u __attribute__((ext_vector_type(2), aligned(4)));
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+
+// v_mfma_f32_32x32x16_f16: lane l supplies A[l % 32][8 (l / 32) + e] and B[8
+// (l / 32) + e][l % 32], e = 0..7; D register r of lane l is D[8 (r / 4) + 4
+// (l / 32) + r % 4][l % 32].
+__device__ __forceinline__ floatx16 mfma32h(half8 a, half8 b, floatx16 c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
+}
+
+// hi and lo fp16 parts of eight values times sc (a power of two)
+__device__ __forceinline__ void split8(const float8v &x, float sc, half8 &h, half8 &l) {
+#pragma unroll
+    for (int e = 0; e < 8; e += 2) {
+        const half2v hh = __builtin_convertvector((float2v{x[e] * sc, x[e + 1] * sc}), half2v);
+        const half2v ll = __builtin_convertvector(
+            (float2v{fmaf(x[e], sc, -(float)hh[0]), fmaf(x[e + 1], sc, -(float)hh[1])}), half2v);
+        h[e] = hh[0];
+        h[e + 1] = hh[1];
+        l[e] = ll[0];
+        l[e + 1] = ll[1];
+    }
+}
+
+// the larger magnitude, NaN if either is
+__device__ __forceinline__ float nmax(float a, float b) { return __builtin_elementwise_maximum(a, b); }
+__device__ __forceinline__ float wave_nmax(float x) {
+    x = nmax(x, dpp<0x128>(x));
+    x = nmax(x, dpp<0x124>(x));
+    x = nmax(x, dpp<0x122>(x));
+    x = nmax(x, dpp<0x121>(x));
+    float a, b;
+    pair16(x, a, b);
+    x = nmax(a, b);
+    pair32(x, a, b);
+    return nmax(a, b);
+}
+__device__ __forceinline__ float pow2(int e) { return __builtin_bit_cast(float, (uint32_t)(e + 127) << 23); }
+// exponent s with max |x| 2^s in [2^13, 2^14), at most 126 (zeros, tiny values)
+__device__ __forceinline__ int scale_exp(float mx) { return mx > 0.f ? min(14 - __builtin_amdgcn_frexp_expf(mx), 126) : 126; }
+__device__ __forceinline__ half8 keep(half8 x, bool finite) {   // x with its finite / non-finite elements, others 0
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const bool f = __builtin_fabsf((float)x[e]) < __builtin_inff();
+        x[e] = f == finite ? x[e] : (_Float16)0.f;
+    }
+    return x;
+}
+
+constexpr int kMfma = 0x8, kDsRead = 0x100;   // __builtin_amdgcn_sched_group_barrier classes
+constexpr int kBK = 32;           // keys per tile
+constexpr int kPShift = 6;        // weights are at most 2^8 times 2^kPShift
+constexpr int kMinB = -60;        // smallest exponent applied to a weight for its V group
+
+// Workgroup = 4 waves of one kv-head g.  The query rows of a kv-head, n_tok
+// positions times n_rep heads, are one list f = z n_rep + i (position major),
+// cut into strips of 32 (a wave) and items of 4 strips (a workgroup): whatever
+// n_rep is, a strip's rows lie within 32 / n_rep + 1 positions, so the waves of
+// a workgroup want the same keys and little is computed for the causal mask to
+// drop.  Per tile of 32 keys a wave computes S^T = K Q^T (keys x queries, 3 hd
+// / 16 MFMAs), so every lane owns the scores of one query; the softmax weights
+// of its 16 keys, split in registers, are the B operand of O^T += V^T P^T (6 hd
+// / 32 MFMAs) without leaving the lane: the k order of the second product is
+// the order in which the first leaves its keys, and V^T is laid out in LDS to
+// match.
+//
+// Tiles: each wave loads a quarter of the next tile (8 keys of K, 8 of V) into
+// registers while the current tile is computed, then scales, splits and writes
+// it to the other LDS buffer, one barrier per tile.  K is kept as chunks of 8
+// dims [hd / 8][33 keys] and V as groups of 8 keys [4][hd], both 16 bytes a
+// unit: an MFMA operand is one 16-byte read, 32 lanes wide and consecutive
+// (no bank conflicts), and the 33rd key spreads the writes of a row's chunks
+// over the banks.  The splits are made once per workgroup, i.e. per 128 query
+// rows; making them in every wave would cost more VALU time than the MFMAs.
+//
+// The softmax runs in base 2 with an integer reference maximum per query (any
+// reference gives the same normalised result): it moves only when the true
+// maximum exceeds it by more than 8, so weights stay below 2^8, the rescale of
+// the accumulators is rare and exact, and the exponent's argument
+// fma(score, scale, offset) has one rounding.
+//
+// HDP: head_dim rounded up to a multiple of 32; EXACT: head_dim == HDP.
+template <int HDP, bool EXACT>
+__global__ __launch_bounds__(kThreads, HDP <= 128 ? 2 : 1) void prefill_kernel(PrefillArgs a) {
+    constexpr int KS = HDP / 16;                    // k-steps of the scores
+    constexpr int NT = HDP / 32;                    // output blocks
+    constexpr int C8 = HDP / 8;                     // 8-dim chunks of a K row
+    constexpr int NUK = (HDP + 63) / 64;            // (key, chunk) units of K per lane
+    constexpr int VD = HDP % 128 == 0 ? 2 : 1;      // dims per V unit
+    constexpr int NUV = (HDP / VD + 63) / 64;
+    constexpr int kKB = C8 * 33 * 16, kVB = 4 * HDP * 16;       // bytes of one part of a tile
+    constexpr int kBuf = 2 * kKB + 2 * kVB + 48;
+    __shared__ __align__(16) unsigned char lds[2 * kBuf];
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int nkv = a.n_head_kv, n_rep = a.n_rep, hd = EXACT ? HDP : a.hd;
+    // work index: items run from the longest (last rows) down; the second part
+    // of the grid takes them from the short end, so that the two workgroups of
+    // a CU (b and b + fold) add up to about the same work
+    const int bx = blockIdx.x;
+    const int wi = bx < a.fold ? bx : (int)gridDim.x - 1 - (bx - a.fold);
+    const int g = wi % nkv;
+    // split plan: unit = item << 2 | part (0 whole, 1 / 2 first / second half)
+    const int unit = a.n_split > 0 ? (int)a.unit[wi / nkv] : 0;
+    const int part = unit & 3;
+    const int seg = a.n_split > 0 ? 0 : (wi / nkv) % a.n_kseg;
+    const int item = a.n_split > 0 ? unit >> 2 : wi / nkv / a.n_kseg;
+    const int F = a.n_tok * n_rep, n_head = nkv * n_rep;
+    const int f0 = kPrefillRows * (a.n_items - 1 - item);        // the item's first row
+    const int n_keys = a.pos0 + a.n_tok;
+    const int wg_kmax = a.pos0 + min(f0 + kPrefillRows - 1, F - 1) / n_rep;
+    const int n_tiles = wg_kmax / kBK + 1;
+    const int ws = f0 + 32 * wave;                               // this wave's first row
+    const int my_kmin = a.pos0 + min(ws, F - 1) / n_rep;         // key limits of its first and last row
+    const int my_kmax = ws < F ? a.pos0 + min(ws + 31, F - 1) / n_rep : -1;
+
+    const int qi = lane & 31, qg = lane >> 5;
+    const int fq = ws + qi;
+    const bool qvalid = fq < F;
+    const int fqc = min(fq, F - 1), qz = fqc / n_rep, qpos = a.pos0 + qz;
+    const size_t qoff = ((size_t)qz * n_head + (size_t)g * n_rep + (fqc - qz * n_rep)) * hd;
+
+    // ---- this wave's share of a tile: keys 8 wave .. + 7 of K as (key, chunk)
+    // units, keys {0..3, 8..11} + 16 (wave / 2) + 4 (wave % 2) of V as dims
+    float8v rk[NUK], rv[NUV][VD];
+    const float *kg = a.kc + (size_t)g * a.slots * hd, *vg = a.vc + (size_t)g * a.slots * hd;
+    const int vkey0 = 16 * (wave >> 1) + 4 * (wave & 1);
+    // rows past the last key repeat it (they are masked): uniform bases, 32-bit lane offsets
+    auto load_tile = [&](int t) {
+        const int k0 = t * kBK, last = n_keys - 1 - k0;
+        const float *kt = kg + (size_t)k0 * hd;
+#pragma unroll
+        for (int i = 0; i < NUK; ++i) {
+            const int u = min(lane + 64 * i, HDP - 1);
+            const unsigned row = __umul24(min(8 * wave + u / C8, last), hd);
+            const int d = 8 * (u % C8);
+            if constexpr (EXACT) {
+                const float4 x = ld4(kt + (row + d)), y = ld4(kt + (row + d + 4));
+                rk[i][0] = x.x; rk[i][1] = x.y; rk[i][2] = x.z; rk[i][3] = x.w;
+                rk[i][4] = y.x; rk[i][5] = y.y; rk[i][6] = y.z; rk[i][7] = y.w;
+            } else {
+#pragma unroll
+                for (int e = 0; e < 8; e += 2) {   // head_dim is even: pairs are whole
+                    const float2 x = *(const float2 *)(kt + (row + min(d + e, hd - 2)));
+                    rk[i][e] = x.x;
+                    rk[i][e + 1] = x.y;
+                }
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const float *vt = vg + (size_t)(k0 + min(vkey0 + (j & 3) + 8 * (j >> 2), last)) * hd;
+#pragma unroll
+            for (int i = 0; i < NUV; ++i) {
+                const unsigned d = VD * min(lane + 64 * i, HDP / VD - 1);
+                if constexpr (VD == 2) {
+                    const float2 x = *(const float2 *)(vt + (EXACT ? d : min(d, (unsigned)hd - 2)));
+                    rv[i][0][j] = x.x;
+                    rv[i][1][j] = x.y;
+                } else {
+                    rv[i][0][j] = vt[EXACT ? d : min(d, (unsigned)hd - 1)];
+                }
+            }
+        }
+    };
+    // dims past head_dim (read from its last ones) count as zeros
+    auto clear_pad = [&] {
+        if constexpr (!EXACT) {
+#pragma unroll
+            for (int i = 0; i < NUK; ++i)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) rk[i][e] = 8 * (min(lane + 64 * i, HDP - 1) % C8) + e < hd ? rk[i][e] : 0.f;
+#pragma unroll
+            for (int i = 0; i < NUV; ++i)
+#pragma unroll
+                for (int d = 0; d < VD; ++d)
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) rv[i][d][j] = VD * (lane + 64 * i) < hd ? rv[i][d][j] : 0.f;
+        }
+    };
+    // scales, splits and writes the loaded share to a buffer, with 2^-scale of
+    // the K group, the scale exponent of the V group and the non-finite flags
+    auto write_tile = [&]<bool SLOW>(int bo) {
+        clear_pad();
+        float mk = 0.f, mv = 0.f;
+#pragma unroll
+        for (int i = 0; i < NUK; ++i)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) mk = nmax(mk, __builtin_fabsf(rk[i][e]));
+#pragma unroll
+        for (int i = 0; i < NUV; ++i)
+#pragma unroll
+            for (int d = 0; d < VD; ++d)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) mv = nmax(mv, __builtin_fabsf(rv[i][d][e]));
+        mk = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, wave_nmax(mk))));
+        mv = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, wave_nmax(mv))));
+        constexpr float kInf = __builtin_inff();
+        const int bad = !(mk < kInf) || !(mv < kInf);    // infinity or NaN
+        if constexpr (SLOW) {                            // the scales of the finite values
+            float fk = 0.f, fv = 0.f;
+#pragma unroll
+            for (int i = 0; i < NUK; ++i)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const float x = __builtin_fabsf(rk[i][e]);
+                    fk = fmaxf(fk, x < kInf ? x : 0.f);
+                }
+#pragma unroll
+            for (int i = 0; i < NUV; ++i)
+#pragma unroll
+                for (int d = 0; d < VD; ++d)
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        const float x = __builtin_fabsf(rv[i][d][e]);
+                        fv = fmaxf(fv, x < kInf ? x : 0.f);
+                    }
+            mk = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, wave_nmax(fk))));
+            mv = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, wave_nmax(fv))));
+        }
+        const int ek = scale_exp(mk), ev = scale_exp(mv);
+        const float sk = pow2(ek), sv = pow2(ev);
+#pragma unroll
+        for (int i = 0; i < NUK; ++i) {
+            const int u = lane + 64 * i;
+            half8 h, l;
+            split8(rk[i], sk, h, l);
+            if constexpr (SLOW) l = keep(l, true);     // inf - inf of a non-finite value
+            if (HDP % 64 == 0 || u < HDP) {
+                unsigned char *p = lds + bo + ((u % C8) * 33 + 8 * wave + u / C8) * 16;
+                *(half8 *)p = h;
+                *(half8 *)(p + kKB) = l;
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < NUV; ++i) {
+            const int u = lane + 64 * i;
+#pragma unroll
+            for (int d = 0; d < VD; ++d) {
+                half8 h, l;
+                split8(rv[i][d], sv, h, l);
+                if constexpr (SLOW) l = keep(l, true);
+                if ((HDP / VD) % 64 == 0 || u < HDP / VD) {
+                    unsigned char *p = lds + bo + 2 * kKB + (wave * HDP + VD * u + d) * 16;
+                    *(half8 *)p = h;
+                    *(half8 *)(p + kVB) = l;
+                }
+            }
+        }
+        if (lane == 0) {
+            float *s = (float *)(lds + bo + 2 * kKB + 2 * kVB);
+            s[wave] = pow2(-ek);
+            ((int *)s)[4 + wave] = ev;
+            ((int *)s)[8 + wave] = bad;
+        }
+    };
+
+    // key tiles of this workgroup: a key segment, a half of a split item
+    // (the plan splits only items of at least two tiles), or all of them
+    const int t_half = n_tiles / 2;
+    const int t_begin = part == 2 ? t_half : seg * a.seg_tiles;
+    const int t_end = part == 1 ? t_half : (a.n_kseg == 1 ? n_tiles : min(n_tiles, t_begin + a.seg_tiles));
+    if (t_begin < t_end) load_tile(t_begin);
+
+    // ---- Q^T operand: roped q of row fq, dims 16 s + 8 qg + e, scaled to the
+    // row's own power of two; cq brings a score to the log2 domain
+    half8 qh[KS], ql[KS];
+    float cq;
+    {
+        float8v y[KS];
+        const float *qp = a.q + qoff;
+        const int half = hd / 2;
+        const float *cs = (const float *)(a.cs + (size_t)qpos * half);
+        float mq = 0.f;
+        if constexpr (EXACT) {                     // dim d + hd / 2 is the same lane's, HDP / 32 steps on
+#pragma unroll
+            for (int s = 0; s < KS / 2; ++s) {
+                const int d = 16 * s + 8 * qg;
+                f4u lo[2], hi[2], c[4];
+#pragma unroll
+                for (int k = 0; k < 2; ++k) {
+                    lo[k] = *(const f4u *)(qp + d + 4 * k);
+                    hi[k] = *(const f4u *)(qp + half + d + 4 * k);
+                }
+#pragma unroll
+                for (int k = 0; k < 4; ++k) c[k] = *(const f4u *)(cs + 2 * d + 4 * k);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    float y0, y1;
+                    rope_pair(lo[e / 4][e % 4], hi[e / 4][e % 4], make_float2(c[e / 2][2 * (e % 2)], c[e / 2][2 * (e % 2) + 1]),
+                              y0, y1);
+                    y[s][e] = y0;
+                    y[s + KS / 2][e] = y1;
+                }
+            }
+        } else {
+#pragma unroll
+            for (int s = 0; s < KS; ++s) {
+                const int d = 16 * s + 8 * qg;
+                const bool low = d + 8 <= half, high = d >= half && d + 8 <= hd;
+                if (low || high) {                 // eight dims on one side of the rotation
+                    const int d0 = low ? d : d - half;
+                    f4u lo[2], hi[2], c[4];
+#pragma unroll
+                    for (int k = 0; k < 2; ++k) {
+                        lo[k] = *(const f4u *)(qp + d0 + 4 * k);
+                        hi[k] = *(const f4u *)(qp + half + d0 + 4 * k);
+                    }
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) c[k] = *(const f4u *)(cs + 2 * d0 + 4 * k);
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        float y0, y1;
+                        rope_pair(lo[e / 4][e % 4], hi[e / 4][e % 4],
+                                  make_float2(c[e / 2][2 * (e % 2)], c[e / 2][2 * (e % 2) + 1]), y0, y1);
+                        y[s][e] = low ? y0 : y1;
+                    }
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        float y0 = 0.f, y1 = 0.f;
+                        if (d + e < hd) {
+                            const int d0 = d + e < half ? d + e : d + e - half;
+                            rope_pair(qp[d0], qp[d0 + half], make_float2(cs[2 * d0], cs[2 * d0 + 1]), y0, y1);
+                        }
+                        y[s][e] = d + e < half ? y0 : y1;
+                    }
+                }
+            }
+        }
+#pragma unroll
+        for (int s = 0; s < KS; ++s)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) mq = fmaxf(mq, __builtin_fabsf(y[s][e]));
+        float ma, mb;
+        pair32(mq, ma, mb);
+        const int eq = scale_exp(fmaxf(ma, mb));   // a non-finite row's scores are NaN whatever the scale
+        const float sq = pow2(eq);
+#pragma unroll
+        for (int s = 0; s < KS; ++s) split8(y[s], sq, qh[s], ql[s]);
+        cq = ldexpf(a.scale_log2, -eq);
+    }
+
+    floatx16 acc[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) acc[t] = floatx16{};
+    float m_run = -INFINITY, l_run = 0.f;          // l_run: this lane's half of the keys
+    int a_ref = 126;                               // acc holds the output times 2^(a_ref + kPShift)
+
+    // SLOW: tiles with infinities or NaN too.  The whole loop exists twice (below),
+    // so that the fast one spends no registers on the other's operands.
+    auto compute_tile = [&]<bool SLOW>(int bo, int t) {
+        const int k0 = t * kBK;
+        if (k0 > my_kmax) return;
+        int ko = bo + (33 * qg + qi) * 16;
+        const unsigned char *vp = lds + bo + 2 * kKB + (qg * HDP + qi) * 16;
+        const float *sp = (const float *)(lds + bo + 2 * kKB + 2 * kVB);
+        const float4 ck = ld4(sp);
+        const int4 av = *(const int4 *)(sp + 4);
+        auto k_at = [&](int st, int part) { return *(const half8 *)(lds + ko + 2 * st * 33 * 16 + part * kKB); };
+        floatx16 s{};
+        double sd[EXACT ? 1 : 16];
+        if constexpr (EXACT && !SLOW) {
+            // the cross terms first: they are small, and the sum then takes one
+            // rounding at its own size per 16 dims
+#pragma unroll
+            for (int st = 0; st < KS; ++st) {
+                s = mfma32h(k_at(st, 0), ql[st], s);
+                s = mfma32h(k_at(st, 1), qh[st], s);
+            }
+            asm volatile("" : "+v"(ko));   // K's hi parts are read again: kept, they would take 2 KS registers too many
+#pragma unroll
+            for (int st = 0; st < KS; ++st) s = mfma32h(k_at(st, 0), qh[st], s);
+            // operands are read a few MFMAs ahead, no further (registers)
+            __builtin_amdgcn_sched_group_barrier(kDsRead, 6, 0);
+#pragma unroll
+            for (int i = 0; i < 3 * KS - 6; ++i) {
+                __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(kDsRead, 1, 0);
+            }
+            __builtin_amdgcn_sched_group_barrier(kMfma, 6, 0);
+        } else if constexpr (EXACT) {
+            // the finite parts as above, then the non-finite ones times hi: inf
+            // times q's sign, NaN for q = 0, as one product gives it
+#pragma unroll
+            for (int st = 0; st < KS; ++st) {
+                s = mfma32h(keep(k_at(st, 0), true), ql[st], s);
+                s = mfma32h(k_at(st, 1), qh[st], s);
+            }
+#pragma unroll
+            for (int st = 0; st < KS; ++st) s = mfma32h(keep(k_at(st, 0), true), qh[st], s);
+#pragma unroll
+            for (int st = 0; st < KS; ++st) s = mfma32h(keep(k_at(st, 0), false), qh[st], s);
+        } else {
+            // 16 dims at a time on the MFMA, lo lo terms included, their sums in fp64
+#pragma unroll
+            for (int st = 0; st < KS; ++st) {
+                const half8 kh = SLOW ? keep(k_at(st, 0), true) : k_at(st, 0), kl = k_at(st, 1);
+                floatx16 x{};
+                x = mfma32h(kl, ql[st], x);
+                x = mfma32h(kh, ql[st], x);
+                x = mfma32h(kl, qh[st], x);
+                x = mfma32h(kh, qh[st], x);
+                if constexpr (SLOW) x = mfma32h(keep(k_at(st, 0), false), qh[st], x);
+#pragma unroll
+                for (int r = 0; r < 16; ++r) sd[r] = st == 0 ? (double)x[r] : sd[r] + (double)x[r];
+            }
+#pragma unroll
+            for (int r = 0; r < 16; ++r) s[r] = (float)sd[r];
+        }
+        // s[r]: query qi, key k0 + 8 (r / 4) + 4 qg + r % 4; the causal mask only
+        // matters on tiles that reach past the strip's first row
+        const float cj[4] = {cq * ck.x, cq * ck.y, cq * ck.z, cq * ck.w};
+        const bool diag = k0 + kBK - 1 > my_kmin;
+        float mt = -INFINITY;
+        if (diag) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                if (k0 + 8 * (r / 4) + 4 * qg + (r % 4) > qpos) {
+                    s[r] = -INFINITY;
+                    if constexpr (!EXACT) sd[r] = -INFINITY;
+                }
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            mt = fmaxf(mt, fmaxf(fmaxf(s[4 * j], s[4 * j + 1]), fmaxf(s[4 * j + 2], s[4 * j + 3])) * cj[j]);
+        {
+            float lo, hi;
+            pair32(mt, lo, hi);
+            mt = fmaxf(lo, hi);
+        }
+        const float m_new = mt > m_run + 8.f ? ceilf(mt) : m_run;
+        const float m_use = m_new == -INFINITY ? 0.f : m_new;    // every key so far masked
+        float alpha = fast_exp2(m_run - m_use);                  // a power of two
+        m_run = m_new;
+        // V groups are scaled apart: acc's units follow the smallest scale so
+        // far, and a group with a larger one takes it from its weights
+        const int av0 = __builtin_amdgcn_readfirstlane(av.x), av1 = __builtin_amdgcn_readfirstlane(av.y);
+        const int av2 = __builtin_amdgcn_readfirstlane(av.z), av3 = __builtin_amdgcn_readfirstlane(av.w);
+        const int a_new = min(a_ref, min(min(av0, av1), min(av2, av3)));
+        const int b0 = max(a_new - (qg ? av1 : av0), kMinB) + kPShift, b1 = max(a_new - (qg ? av3 : av2), kMinB) + kPShift;
+        const float nm0 = (float)b0 - m_use, nm1 = (float)b1 - m_use;
+        float ps0 = 0.f, ps1 = 0.f;
+        half8 ph[2], pl[2];
+        {
+            float8v p0, p1;
+#pragma unroll
+            for (int r = 0; r < 8; ++r) {
+                if constexpr (EXACT) {
+                    p0[r] = fast_exp2(fmaf(s[r], cj[r / 4], nm0));
+                    p1[r] = fast_exp2(fmaf(s[8 + r], cj[2 + r / 4], nm1));
+                } else {
+                    p0[r] = fast_exp2((float)fma(sd[r], (double)cj[r / 4], (double)nm0));
+                    p1[r] = fast_exp2((float)fma(sd[8 + r], (double)cj[2 + r / 4], (double)nm1));
+                }
+                ps0 += p0[r];
+                ps1 += p1[r];
+            }
+            split8(p0, 1.f, ph[0], pl[0]);
+            split8(p1, 1.f, ph[1], pl[1]);
+        }
+        l_run = fmaf(l_run, alpha, ldexpf(ps0, -b0) + ldexpf(ps1, -b1));
+        if (a_new != a_ref) alpha = ldexpf(alpha, a_new - a_ref);
+        a_ref = a_new;
+        // rescale only when some query's reference (or the V scale) moved
+        if (__builtin_amdgcn_ballot_w64(alpha != 1.f)) {
+#pragma unroll
+            for (int tt = 0; tt < NT; ++tt)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc[tt][r] *= alpha;
+        }
+        if constexpr (!SLOW) {
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+                for (int tt = 0; tt < NT; ++tt) {
+                    const half8 vh = *(const half8 *)(vp + (2 * ks * HDP + 32 * tt) * 16);
+                    const half8 vl = *(const half8 *)(vp + (2 * ks * HDP + 32 * tt) * 16 + kVB);
+                    acc[tt] = mfma32h(vl, ph[ks], acc[tt]);
+                    acc[tt] = mfma32h(vh, pl[ks], acc[tt]);
+                    acc[tt] = mfma32h(vh, ph[ks], acc[tt]);
+                }
+            __builtin_amdgcn_sched_group_barrier(kDsRead, 4, 1);
+#pragma unroll
+            for (int i = 0; i < 2 * NT - 2; ++i) {
+                __builtin_amdgcn_sched_group_barrier(kMfma, 3, 1);
+                __builtin_amdgcn_sched_group_barrier(kDsRead, 2, 1);
+            }
+            __builtin_amdgcn_sched_group_barrier(kMfma, 6, 1);
+        } else {
+            // the finite parts as above; of the non-finite ones, how many +inf,
+            // -inf and NaN every (query, dim) gets from keys it attends (a weight
+            // of 0 for a masked key must not make NaN of them)
+            half8 on[2];
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                on[r / 8][r % 8] = k0 + 8 * (r / 4) + 4 * qg + (r % 4) <= qpos ? (_Float16)1.f : (_Float16)0.f;
+#pragma unroll
+            for (int tt = 0; tt < NT; ++tt) {
+#pragma unroll
+                for (int ks = 0; ks < 2; ++ks) {
+                    const half8 vh = keep(*(const half8 *)(vp + (2 * ks * HDP + 32 * tt) * 16), true);
+                    const half8 vl = *(const half8 *)(vp + (2 * ks * HDP + 32 * tt) * 16 + kVB);
+                    acc[tt] = mfma32h(vl, ph[ks], acc[tt]);
+                    acc[tt] = mfma32h(vh, pl[ks], acc[tt]);
+                    acc[tt] = mfma32h(vh, ph[ks], acc[tt]);
+                }
+                auto count = [&](auto is, float add) {
+                    floatx16 n{};
+#pragma unroll
+                    for (int ks = 0; ks < 2; ++ks) {
+                        const half8 v8 = *(const half8 *)(vp + (2 * ks * HDP + 32 * tt) * 16);
+                        half8 c;
+#pragma unroll
+                        for (int e = 0; e < 8; ++e) c[e] = is((float)v8[e]) ? (_Float16)1.f : (_Float16)0.f;
+                        n = mfma32h(c, on[ks], n);
+                    }
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) acc[tt][r] += n[r] > 0.f ? add : 0.f;
+                    __builtin_amdgcn_sched_barrier(0);
+                };
+                count([](float x) { return x == __builtin_inff(); }, __builtin_inff());
+                count([](float x) { return x == -__builtin_inff(); }, -__builtin_inff());
+                count([](float x) { return x != x; }, __builtin_nanf(""));
+            }
+        }
+    };
+
+    // false if a tile has infinities or NaN and SLOW is not set (the loads of the
+    // tiles after it are then dropped)
+    auto run = [&]<bool SLOW>() {
+        for (int t = t_begin - 1; t < t_end; ++t) {            // one turn ahead: the first tile's write
+            const int bo = ((t - t_begin) & 1) * kBuf;
+            if (t >= t_begin) {
+                if constexpr (!SLOW) {
+                    const int4 bv = *(const int4 *)(lds + bo + 2 * kKB + 2 * kVB + 32);
+                    if (__builtin_amdgcn_readfirstlane(bv.x | bv.y | bv.z | bv.w)) return false;   // the same in every wave
+                }
+                compute_tile.template operator()<SLOW>(bo, t);
+            }
+            if (t + 1 < t_end) {
+                write_tile.template operator()<SLOW>(kBuf - bo);
+                if (t + 2 < t_end) load_tile(t + 2);
+            }
+            __syncthreads();
+        }
+        return true;
+    };
+    if (!run.template operator()<false>()) {
+        __syncthreads();                            // every wave has left the fast loop's buffers
+#pragma unroll
+        for (int tt = 0; tt < NT; ++tt) acc[tt] = floatx16{};
+        m_run = -INFINITY;
+        l_run = 0.f;
+        a_ref = 126;
+        load_tile(t_begin);
+        run.template operator()<true>();
+    }
+
+    // output: lane (qi, qg) register r of block tt is dim 32 tt + 8 (r / 4) + 4 qg + r % 4
+    {
+        float lo, hi;
+        pair32(l_run, lo, hi);
+        l_run = lo + hi;
+    }
+    const int sh = -(a_ref + kPShift);
+    if (a.n_kseg > 1 || part != 0) {
+        if (ws >= F) return;
+        const size_t pe = part != 0 ? (((size_t)g * a.n_split + item) * 4 + wave) * 2 + (part - 1)
+                                    : (((size_t)g * a.n_items + item) * 4 + wave) * a.n_kseg + seg;
+        float *dst = a.part_o + (pe * 32 + qi) * HDP;
+#pragma unroll
+        for (int tt = 0; tt < NT; ++tt)
+#pragma unroll
+            for (int r = 0; r < 16; r += 4)
+                st4(dst + 32 * tt + 2 * r + 4 * qg, make_float4(ldexpf(acc[tt][r], sh), ldexpf(acc[tt][r + 1], sh),
+                                                                ldexpf(acc[tt][r + 2], sh), ldexpf(acc[tt][r + 3], sh)));
+        if (qg == 0) {
+            a.part_ml[(pe * 32 + qi) * 2 + 0] = m_run;
+            a.part_ml[(pe * 32 + qi) * 2 + 1] = l_run;
+        }
+        return;
+    }
+    if (!qvalid) return;
+    const float inv = 1.f / l_run;
+    float *dst = a.out + qoff;
+#pragma unroll
+    for (int tt = 0; tt < NT; ++tt)
+#pragma unroll
+        for (int r = 0; r < 16; r += 4) {
+            const int d = 32 * tt + 2 * r + 4 * qg;
+            float x[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[e] = ldexpf(acc[tt][r + e] * inv, sh);
+            if (EXACT || d + 4 <= hd) *(f4u *)(dst + d) = f4u{x[0], x[1], x[2], x[3]};
+            else if (d + 2 <= hd) *(f2u *)(dst + d) = f2u{x[0], x[1]};
+        }
+}
+
+// Block = 32 query rows of one strip of a kv-head: the log-sum-exp merge of the
+// key segments (or of the two halves of a split item); thread (row tid / 8, c =
+// tid % 8) owns the float4s c, c + 8, ... of its row.  Segments in batches of
+// four, every load of a batch issued before its arithmetic (one memory round
+// trip per batch).
+template <int HDP, bool EXACT>
+__global__ __launch_bounds__(256) void prefill_combine_kernel(PrefillArgs a) {
+    constexpr int N4 = HDP / 32;                        // float4 per thread
+    const int hd = EXACT ? HDP : a.hd, F = a.n_tok * a.n_rep;
+    int g, item;
+    const int id = blockIdx.x, gi = id >> 2, wave = id & 3;
+    const int S = a.n_split > 0 ? 2 : a.n_kseg;
+    const int per = a.n_split > 0 ? a.n_split : a.n_items;
+    g = gi / per;
+    item = gi - g * per;
+    const size_t base = (size_t)id * S;
+    const int r = threadIdx.x >> 3, c = threadIdx.x & 7;
+    const int f = kPrefillRows * (a.n_items - 1 - item) + 32 * wave + r;
+    if (f >= F) return;
+    constexpr int kSeg = 4;
+    const float2 *ml = reinterpret_cast<const float2 *>(a.part_ml);
+    float m = -INFINITY;
+    for (int s0 = 0; s0 < S; s0 += 2 * kSeg) {
+        float mv[2 * kSeg];
+#pragma unroll
+        for (int u = 0; u < 2 * kSeg; ++u) mv[u] = s0 + u < S ? ml[(base + s0 + u) * 32 + r].x : -INFINITY;
+#pragma unroll
+        for (int u = 0; u < 2 * kSeg; ++u) m = fmaxf(m, mv[u]);
+    }
+    float den = 0.f;
+    float4 acc[N4];
+#pragma unroll
+    for (int j = 0; j < N4; ++j) acc[j] = zero4();
+    for (int s0 = 0; s0 < S; s0 += kSeg) {
+        float2 st[kSeg];
+        float4 x[kSeg][N4];
+#pragma unroll
+        for (int u = 0; u < kSeg; ++u)
+            if (s0 + u < S) {
+                st[u] = ml[(base + s0 + u) * 32 + r];
+                const float *po = a.part_o + ((base + s0 + u) * 32 + r) * HDP + 4 * c;
+#pragma unroll
+                for (int j = 0; j < N4; ++j) x[u][j] = ld4(po + 32 * j);
+            }
+#pragma unroll
+        for (int u = 0; u < kSeg; ++u)
+            if (s0 + u < S && st[u].x != -INFINITY) {       // a segment may hold masked keys only
+                const float w = exp2f(st[u].x - m);
+                den = fmaf(w, st[u].y, den);
+#pragma unroll
+                for (int j = 0; j < N4; ++j) {
+                    acc[j].x = fmaf(w, x[u][j].x, acc[j].x);
+                    acc[j].y = fmaf(w, x[u][j].y, acc[j].y);
+                    acc[j].z = fmaf(w, x[u][j].z, acc[j].z);
+                    acc[j].w = fmaf(w, x[u][j].w, acc[j].w);
+                }
+            }
+    }
+    const float inv = 1.f / den;
+    const int z = f / a.n_rep;
+    float *op = a.out + ((size_t)z * a.n_head_kv * a.n_rep + (size_t)g * a.n_rep + (f - z * a.n_rep)) * hd;
+#pragma unroll
+    for (int j = 0; j < N4; ++j) {
+        const int d = 32 * j + 4 * c;
+        if (EXACT || d + 4 <= hd) *(f4u *)(op + d) = f4u{acc[j].x * inv, acc[j].y * inv, acc[j].z * inv, acc[j].w * inv};
+        else if (d + 2 <= hd) *(f2u *)(op + d) = f2u{acc[j].x * inv, acc[j].y * inv};
+    }
+}
+
+// ---------------------------------------------------------------- dispatch
+
+int per_cu(int head_dim) { return head_dim <= 128 ? 2 : 1; }   // workgroups that fit a CU
+
+template <int HDP, bool EXACT>
+hipError_t launch_t(const PrefillArgs &a, hipStream_t s) {
+    const dim3 grid(a.n_split > 0 ? a.n_units * a.n_head_kv : a.n_items * a.n_head_kv * a.n_kseg);
+    hipLaunchKernelGGL((prefill_kernel<HDP, EXACT>), grid, dim3(kThreads), 0, s, a);
+    if (a.n_split > 0 || a.n_kseg > 1) {
+        const dim3 cgrid(a.n_head_kv * (a.n_split > 0 ? a.n_split : a.n_items) * 4);
+        hipLaunchKernelGGL((prefill_combine_kernel<HDP, EXACT>), cgrid, dim3(256), 0, s, a);
+    }
+    return hipGetLastError();
+}
+
+}  // namespace
+
+int prefill_padded_dim(int head_dim) { return (head_dim + 31) / 32 * 32; }
+
+size_t prefill_part_floats(int head_dim, int num_cu) {
+    return (size_t)2 * num_cu * kPrefillRows * (prefill_padded_dim(head_dim) + 2);
+}
+
+void prefill_plan(PrefillArgs &a, int num_cu) {
+    a.n_items = (a.n_tok * a.n_rep + kPrefillRows - 1) / kPrefillRows;
+    a.n_split = 0;
+    a.n_units = 0;
+    a.n_kseg = 1;
+    a.fold = num_cu;
+    const int cu = per_cu(a.hd), n_wg = a.n_items * a.n_head_kv, F = a.n_tok * a.n_rep;
+    auto tiles = [&](int i) {   // key tiles of item i (its last row)
+        const int f0 = kPrefillRows * (a.n_items - 1 - i);
+        return (a.pos0 + std::min(f0 + kPrefillRows - 1, F - 1) / a.n_rep) / kBK + 1;
+    };
+    // Split the key range when the workgroups of a chunk do not fill every
+    // CU: as many segments as keep all of them in one wave, each of at least
+    // 2 key tiles.  A 64-row chunk has 16 workgroups (7B): unsplit, each walks
+    // all its key tiles alone.
+    if (n_wg < num_cu) a.n_kseg = std::max(1, std::min(cu * num_cu / n_wg, tiles(0) / 2));
+    a.seg_tiles = (tiles(0) + a.n_kseg - 1) / a.n_kseg;
+    // Two workgroups fit per CU and the grid is folded so that each CU's pair
+    // adds up to about the mean work; with between one and two workgroups per
+    // CU some CUs hold one item only, while the pairs' sums run up to about
+    // the longest item plus the shortest.  Splitting the longest items into
+    // two halves of their key tiles fills the grid to two per CU and lets the
+    // pairs (r-th longest unit with the r-th shortest) even out.
+    if (a.n_kseg != 1 || n_wg < num_cu || n_wg >= cu * num_cu) return;
+    int split = std::min(a.n_items, (cu * num_cu - n_wg) / a.n_head_kv);
+    while (split > 0 && tiles(split - 1) < 4) --split;   // halves of at least two tiles
+    if (split == 0 || a.n_items + split > kMaxPrefillUnits) return;
+    struct Unit { int tiles, code; };
+    std::vector<Unit> u;
+    u.reserve(a.n_items + split);
+    for (int i = 0; i < a.n_items; ++i) {
+        const int t = tiles(i);
+        if (i < split) {
+            u.push_back({t / 2, i << 2 | 1});
+            u.push_back({t - t / 2, i << 2 | 2});
+        } else {
+            u.push_back({t, i << 2});
+        }
+    }
+    std::stable_sort(u.begin(), u.end(), [](const Unit &x, const Unit &y) { return x.tiles > y.tiles; });
+    for (size_t r = 0; r < u.size(); ++r) a.unit[r] = (uint16_t)u[r].code;
+    a.n_split = split;
+    a.n_units = (int)u.size();
+}
+
+hipError_t launch_prefill(const PrefillArgs &a, hipStream_t s) {
+    switch (prefill_padded_dim(a.hd)) {
+        case 32: return launch_t<32, false>(a, s);
+        case 64: return a.hd == 64 ? launch_t<64, true>(a, s) : launch_t<64, false>(a, s);
+        case 96: return launch_t<96, false>(a, s);
+        case 128: return a.hd == 128 ? launch_t<128, true>(a, s) : launch_t<128, false>(a, s);
+        case 160: return launch_t<160, false>(a, s);
+        case 192: return launch_t<192, false>(a, s);
+        case 224: return launch_t<224, false>(a, s);
+        case 256: return launch_t<256, false>(a, s);
+        default: return hipErrorInvalidValue;
+    }
+}
+
+}  // namespace kore_attn_gpu
