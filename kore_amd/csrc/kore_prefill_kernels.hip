@@ -10,20 +10,22 @@
 //
 // Why split fp16.  The fp32 matrix rate (157 TFLOP/s) bounds the two products;
 // fp16 runs 16 times as fast, and x = hi + lo with hi = fp16(x), lo = fp16(x -
-// hi) carries 22 bits, so three products (hi hi + hi lo + lo hi, each exact,
+// hi) carries 23 of 24 bits, so three products (hi hi + hi lo + lo hi, each exact,
 // summed in fp32) cost 3 / 16 of the fp32 ones.  The sums take 16 products per
 // fp32 rounding instead of two, and the score's small cross terms are summed
 // first, so the result is nearer to the exact one than the fp32 kernel's was
 // (28/4/128, 2048 rows: 3.9e-7 of the 2-norm against 7.2e-7).  A head_dim that
-// is neither 64 nor 128 ran on VALU with fp64 scores; to lose nothing there its
-// scores take the fourth product and sum their 16-dim pieces in fp64 (33/3/96,
-// 700 rows: 3.6e-7 both; 4/4/140: 2.0e-7 against 1.8e-7 and 2.1e-7).
+// is neither 64 nor 128 ran on VALU with fp64 scores; to lose nothing there a
+// third part holds the last bit (six products) and the scores' 16-dim pieces
+// are summed in fp64 (33/3/96, 700 rows: 2.8e-7 against 4.0e-7; 4/4/140, 175
+// rows: 1.4e-7 against 1.8e-7).
 //
 // Measured, one layer, against the kernels before (fp32 MFMA; VALU for 33/3/96):
 // 28/4/128 2048 rows 261 -> 141 us (114 -> 213 TFLOP/s), 12/2/128 333 rows at
-// 7001 151 -> 73 us, 33/3/96 700 rows at 100 731 -> 54 us.  What bounds it now:
-// the MFMAs (39 % of the cycles) and the softmax and split arithmetic (47 %)
-// hardly overlap, since a wave does one after the other.
+// 7001 151 -> 73 us, 33/3/96 700 rows at 100 731 -> 81 us (101 with one
+// workgroup per CU; two parts with fp64 sums 54 us, but 4/4/140 at 2.0e-7).
+// What bounds it now: the MFMAs (39 % of the cycles) and the softmax and split
+// arithmetic (47 %) hardly overlap, since a wave does one after the other.
 //
 // Range.  fp16 holds 2^-24 .. 65504, so every operand is scaled by a power of
 // two (exact) that brings its largest magnitude to 2^13 .. 2^14: a query row
@@ -55,17 +57,24 @@ __device__ __forceinline__ floatx16 mfma32h(half8 a, half8 b, floatx16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
 }
 
-// hi and lo fp16 parts of eight values times sc (a power of two)
-__device__ __forceinline__ void split8(const float8v &x, float sc, half8 &h, half8 &l) {
+// the fp16 parts of eight values times sc (a power of two), PARTS of them: hi,
+// lo and what those two leave (one bit of 24)
+template <int PARTS>
+__device__ __forceinline__ void split8(const float8v &x, float sc, half8 *p) {
 #pragma unroll
     for (int e = 0; e < 8; e += 2) {
-        const half2v hh = __builtin_convertvector((float2v{x[e] * sc, x[e + 1] * sc}), half2v);
-        const half2v ll = __builtin_convertvector(
-            (float2v{fmaf(x[e], sc, -(float)hh[0]), fmaf(x[e + 1], sc, -(float)hh[1])}), half2v);
-        h[e] = hh[0];
-        h[e + 1] = hh[1];
-        l[e] = ll[0];
-        l[e + 1] = ll[1];
+        const half2v h = __builtin_convertvector((float2v{x[e] * sc, x[e + 1] * sc}), half2v);
+        const float r0 = fmaf(x[e], sc, -(float)h[0]), r1 = fmaf(x[e + 1], sc, -(float)h[1]);
+        const half2v l = __builtin_convertvector((float2v{r0, r1}), half2v);
+        p[0][e] = h[0];
+        p[0][e + 1] = h[1];
+        p[1][e] = l[0];
+        p[1][e + 1] = l[1];
+        if constexpr (PARTS == 3) {
+            const half2v r = __builtin_convertvector((float2v{r0 - (float)l[0], r1 - (float)l[1]}), half2v);
+            p[2][e] = r[0];
+            p[2][e + 1] = r[1];
+        }
     }
 }
 
@@ -94,6 +103,9 @@ __device__ __forceinline__ half8 keep(half8 x, bool finite) {   // x with its fi
     return x;
 }
 
+// workgroups of prefill_kernel that fit a CU (registers, LDS)
+constexpr int per_cu(int hdp, bool exact) { return hdp <= (exact ? 128 : 96) ? 2 : 1; }
+
 constexpr int kMfma = 0x8, kDsRead = 0x100;   // __builtin_amdgcn_sched_group_barrier classes
 constexpr int kBK = 32;           // keys per tile
 constexpr int kPShift = 6;        // weights are at most 2^8 times 2^kPShift
@@ -120,15 +132,18 @@ constexpr int kMinB = -60;        // smallest exponent applied to a weight for i
 // over the banks.  The splits are made once per workgroup, i.e. per 128 query
 // rows; making them in every wave would cost more VALU time than the MFMAs.
 //
-// The softmax runs in base 2 with an integer reference maximum per query (any
-// reference gives the same normalised result): it moves only when the true
-// maximum exceeds it by more than 8, so weights stay below 2^8, the rescale of
-// the accumulators is rare and exact, and the exponent's argument
-// fma(score, scale, offset) has one rounding.
+// The softmax runs in base 2.  EXACT keeps an integer reference maximum per
+// query (any reference gives the same normalised result) that moves only when
+// the true maximum exceeds it by more than 8, so weights stay below 2^8 and the
+// rescale of the accumulators is rare and exact; otherwise the reference is the
+// maximum itself, whose weight is then 1.  The exponent's argument fma(score,
+// scale, -reference) has one rounding.
 //
-// HDP: head_dim rounded up to a multiple of 32; EXACT: head_dim == HDP.
+// HDP: head_dim rounded up to a multiple of 32.  EXACT (head_dim == HDP, 64 or
+// 128): two fp16 parts per operand, 23 of 24 bits; otherwise three, the whole
+// fp32 value, scores summed in fp64 and each tile's output summed apart.
 template <int HDP, bool EXACT>
-__global__ __launch_bounds__(kThreads, HDP <= 128 ? 2 : 1) void prefill_kernel(PrefillArgs a) {
+__global__ __launch_bounds__(kThreads, per_cu(HDP, EXACT)) void prefill_kernel(PrefillArgs a) {
     constexpr int KS = HDP / 16;                    // k-steps of the scores
     constexpr int NT = HDP / 32;                    // output blocks
     constexpr int C8 = HDP / 8;                     // 8-dim chunks of a K row
@@ -136,8 +151,10 @@ __global__ __launch_bounds__(kThreads, HDP <= 128 ? 2 : 1) void prefill_kernel(P
     constexpr int VD = HDP % 128 == 0 ? 2 : 1;      // dims per V unit
     constexpr int NUV = (HDP / VD + 63) / 64;
     constexpr int kKB = C8 * 33 * 16, kVB = 4 * HDP * 16;       // bytes of one part of a tile
-    constexpr int kBuf = 2 * kKB + 2 * kVB + 48;
-    __shared__ __align__(16) unsigned char lds[2 * kBuf];
+    constexpr int PARTS = EXACT ? 2 : 3;            // fp16 parts of an operand
+    constexpr int kVOff = PARTS * kKB, kMeta = PARTS * (kKB + kVB), kBuf = kMeta + 48;
+    constexpr int NBUF = 2 * kBuf <= 160 * 1024 ? 2 : 1;
+    __shared__ __align__(16) unsigned char lds[NBUF * kBuf];
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -271,32 +288,32 @@ __global__ __launch_bounds__(kThreads, HDP <= 128 ? 2 : 1) void prefill_kernel(P
 #pragma unroll
         for (int i = 0; i < NUK; ++i) {
             const int u = lane + 64 * i;
-            half8 h, l;
-            split8(rk[i], sk, h, l);
-            if constexpr (SLOW) l = keep(l, true);     // inf - inf of a non-finite value
-            if (HDP % 64 == 0 || u < HDP) {
-                unsigned char *p = lds + bo + ((u % C8) * 33 + 8 * wave + u / C8) * 16;
-                *(half8 *)p = h;
-                *(half8 *)(p + kKB) = l;
-            }
+            half8 h[PARTS];
+            split8<PARTS>(rk[i], sk, h);
+#pragma unroll
+            for (int q = 1; SLOW && q < PARTS; ++q) h[q] = keep(h[q], true);   // inf - inf of a non-finite value
+            if (HDP % 64 == 0 || u < HDP)
+#pragma unroll
+                for (int q = 0; q < PARTS; ++q)
+                    *(half8 *)(lds + bo + q * kKB + ((u % C8) * 33 + 8 * wave + u / C8) * 16) = h[q];
         }
 #pragma unroll
         for (int i = 0; i < NUV; ++i) {
             const int u = lane + 64 * i;
 #pragma unroll
             for (int d = 0; d < VD; ++d) {
-                half8 h, l;
-                split8(rv[i][d], sv, h, l);
-                if constexpr (SLOW) l = keep(l, true);
-                if ((HDP / VD) % 64 == 0 || u < HDP / VD) {
-                    unsigned char *p = lds + bo + 2 * kKB + (wave * HDP + VD * u + d) * 16;
-                    *(half8 *)p = h;
-                    *(half8 *)(p + kVB) = l;
-                }
+                half8 h[PARTS];
+                split8<PARTS>(rv[i][d], sv, h);
+#pragma unroll
+                for (int q = 1; SLOW && q < PARTS; ++q) h[q] = keep(h[q], true);
+                if ((HDP / VD) % 64 == 0 || u < HDP / VD)
+#pragma unroll
+                    for (int q = 0; q < PARTS; ++q)
+                        *(half8 *)(lds + bo + kVOff + q * kVB + (wave * HDP + VD * u + d) * 16) = h[q];
             }
         }
         if (lane == 0) {
-            float *s = (float *)(lds + bo + 2 * kKB + 2 * kVB);
+            float *s = (float *)(lds + bo + kMeta);
             s[wave] = pow2(-ek);
             ((int *)s)[4 + wave] = ev;
             ((int *)s)[8 + wave] = bad;
@@ -312,7 +329,7 @@ __global__ __launch_bounds__(kThreads, HDP <= 128 ? 2 : 1) void prefill_kernel(P
 
     // ---- Q^T operand: roped q of row fq, dims 16 s + 8 qg + e, scaled to the
     // row's own power of two; cq brings a score to the log2 domain
-    half8 qh[KS], ql[KS];
+    half8 qp8[KS][PARTS];
     float cq;
     {
         float8v y[KS];
@@ -385,7 +402,7 @@ __global__ __launch_bounds__(kThreads, HDP <= 128 ? 2 : 1) void prefill_kernel(P
         const int eq = scale_exp(fmaxf(ma, mb));   // a non-finite row's scores are NaN whatever the scale
         const float sq = pow2(eq);
 #pragma unroll
-        for (int s = 0; s < KS; ++s) split8(y[s], sq, qh[s], ql[s]);
+        for (int s = 0; s < KS; ++s) split8<PARTS>(y[s], sq, qp8[s]);
         cq = ldexpf(a.scale_log2, -eq);
     }
 
@@ -401,8 +418,8 @@ __global__ __launch_bounds__(kThreads, HDP <= 128 ? 2 : 1) void prefill_kernel(P
         const int k0 = t * kBK;
         if (k0 > my_kmax) return;
         int ko = bo + (33 * qg + qi) * 16;
-        const unsigned char *vp = lds + bo + 2 * kKB + (qg * HDP + qi) * 16;
-        const float *sp = (const float *)(lds + bo + 2 * kKB + 2 * kVB);
+        const unsigned char *vp = lds + bo + kVOff + (qg * HDP + qi) * 16;
+        const float *sp = (const float *)(lds + bo + kMeta);
         const float4 ck = ld4(sp);
         const int4 av = *(const int4 *)(sp + 4);
         auto k_at = [&](int st, int part) { return *(const half8 *)(lds + ko + 2 * st * 33 * 16 + part * kKB); };
@@ -413,12 +430,12 @@ __global__ __launch_bounds__(kThreads, HDP <= 128 ? 2 : 1) void prefill_kernel(P
             // rounding at its own size per 16 dims
 #pragma unroll
             for (int st = 0; st < KS; ++st) {
-                s = mfma32h(k_at(st, 0), ql[st], s);
-                s = mfma32h(k_at(st, 1), qh[st], s);
+                s = mfma32h(k_at(st, 0), qp8[st][1], s);
+                s = mfma32h(k_at(st, 1), qp8[st][0], s);
             }
             asm volatile("" : "+v"(ko));   // K's hi parts are read again: kept, they would take 2 KS registers too many
 #pragma unroll
-            for (int st = 0; st < KS; ++st) s = mfma32h(k_at(st, 0), qh[st], s);
+            for (int st = 0; st < KS; ++st) s = mfma32h(k_at(st, 0), qp8[st][0], s);
             // operands are read a few MFMAs ahead, no further (registers)
             __builtin_amdgcn_sched_group_barrier(kDsRead, 6, 0);
 #pragma unroll
@@ -432,24 +449,26 @@ __global__ __launch_bounds__(kThreads, HDP <= 128 ? 2 : 1) void prefill_kernel(P
             // times q's sign, NaN for q = 0, as one product gives it
 #pragma unroll
             for (int st = 0; st < KS; ++st) {
-                s = mfma32h(keep(k_at(st, 0), true), ql[st], s);
-                s = mfma32h(k_at(st, 1), qh[st], s);
+                s = mfma32h(keep(k_at(st, 0), true), qp8[st][1], s);
+                s = mfma32h(k_at(st, 1), qp8[st][0], s);
             }
 #pragma unroll
-            for (int st = 0; st < KS; ++st) s = mfma32h(keep(k_at(st, 0), true), qh[st], s);
+            for (int st = 0; st < KS; ++st) s = mfma32h(keep(k_at(st, 0), true), qp8[st][0], s);
 #pragma unroll
-            for (int st = 0; st < KS; ++st) s = mfma32h(keep(k_at(st, 0), false), qh[st], s);
+            for (int st = 0; st < KS; ++st) s = mfma32h(keep(k_at(st, 0), false), qp8[st][0], s);
         } else {
-            // 16 dims at a time on the MFMA, lo lo terms included, their sums in fp64
+            // 16 dims at a time on the MFMA, to 2^-24 of the operands, their sums in fp64
 #pragma unroll
             for (int st = 0; st < KS; ++st) {
-                const half8 kh = SLOW ? keep(k_at(st, 0), true) : k_at(st, 0), kl = k_at(st, 1);
+                const half8 kh = SLOW ? keep(k_at(st, 0), true) : k_at(st, 0), kl = k_at(st, 1), kr = k_at(st, 2);
                 floatx16 x{};
-                x = mfma32h(kl, ql[st], x);
-                x = mfma32h(kh, ql[st], x);
-                x = mfma32h(kl, qh[st], x);
-                x = mfma32h(kh, qh[st], x);
-                if constexpr (SLOW) x = mfma32h(keep(k_at(st, 0), false), qh[st], x);
+                x = mfma32h(kr, qp8[st][0], x);
+                x = mfma32h(kh, qp8[st][2], x);
+                x = mfma32h(kl, qp8[st][1], x);
+                x = mfma32h(kl, qp8[st][0], x);
+                x = mfma32h(kh, qp8[st][1], x);
+                x = mfma32h(kh, qp8[st][0], x);
+                if constexpr (SLOW) x = mfma32h(keep(k_at(st, 0), false), qp8[st][0], x);
 #pragma unroll
                 for (int r = 0; r < 16; ++r) sd[r] = st == 0 ? (double)x[r] : sd[r] + (double)x[r];
             }
@@ -477,9 +496,9 @@ __global__ __launch_bounds__(kThreads, HDP <= 128 ? 2 : 1) void prefill_kernel(P
             pair32(mt, lo, hi);
             mt = fmaxf(lo, hi);
         }
-        const float m_new = mt > m_run + 8.f ? ceilf(mt) : m_run;
+        const float m_new = EXACT ? (mt > m_run + 8.f ? ceilf(mt) : m_run) : fmaxf(m_run, mt);
         const float m_use = m_new == -INFINITY ? 0.f : m_new;    // every key so far masked
-        float alpha = fast_exp2(m_run - m_use);                  // a power of two
+        float alpha = fast_exp2(m_run - m_use);                  // EXACT: a power of two
         m_run = m_new;
         // V groups are scaled apart: acc's units follow the smallest scale so
         // far, and a group with a larger one takes it from its weights
@@ -487,27 +506,26 @@ __global__ __launch_bounds__(kThreads, HDP <= 128 ? 2 : 1) void prefill_kernel(P
         const int av2 = __builtin_amdgcn_readfirstlane(av.z), av3 = __builtin_amdgcn_readfirstlane(av.w);
         const int a_new = min(a_ref, min(min(av0, av1), min(av2, av3)));
         const int b0 = max(a_new - (qg ? av1 : av0), kMinB) + kPShift, b1 = max(a_new - (qg ? av3 : av2), kMinB) + kPShift;
-        const float nm0 = (float)b0 - m_use, nm1 = (float)b1 - m_use;
-        float ps0 = 0.f, ps1 = 0.f;
-        half8 ph[2], pl[2];
+        // near 0 for the keys that count, so that its rounding is small
+        float ps = 0.f;
+        half8 pp[2][PARTS];
         {
             float8v p0, p1;
 #pragma unroll
             for (int r = 0; r < 8; ++r) {
                 if constexpr (EXACT) {
-                    p0[r] = fast_exp2(fmaf(s[r], cj[r / 4], nm0));
-                    p1[r] = fast_exp2(fmaf(s[8 + r], cj[2 + r / 4], nm1));
+                    p0[r] = fast_exp2(fmaf(s[r], cj[r / 4], -m_use));
+                    p1[r] = fast_exp2(fmaf(s[8 + r], cj[2 + r / 4], -m_use));
                 } else {
-                    p0[r] = fast_exp2((float)fma(sd[r], (double)cj[r / 4], (double)nm0));
-                    p1[r] = fast_exp2((float)fma(sd[8 + r], (double)cj[2 + r / 4], (double)nm1));
+                    p0[r] = fast_exp2((float)fma(sd[r], (double)cj[r / 4], (double)-m_use));
+                    p1[r] = fast_exp2((float)fma(sd[8 + r], (double)cj[2 + r / 4], (double)-m_use));
                 }
-                ps0 += p0[r];
-                ps1 += p1[r];
+                ps += p0[r] + p1[r];
             }
-            split8(p0, 1.f, ph[0], pl[0]);
-            split8(p1, 1.f, ph[1], pl[1]);
+            split8<PARTS>(p0, pow2(b0), pp[0]);
+            split8<PARTS>(p1, pow2(b1), pp[1]);
         }
-        l_run = fmaf(l_run, alpha, ldexpf(ps0, -b0) + ldexpf(ps1, -b1));
+        l_run = fmaf(l_run, alpha, ps);
         if (a_new != a_ref) alpha = ldexpf(alpha, a_new - a_ref);
         a_ref = a_new;
         // rescale only when some query's reference (or the V scale) moved
@@ -517,17 +535,33 @@ __global__ __launch_bounds__(kThreads, HDP <= 128 ? 2 : 1) void prefill_kernel(P
 #pragma unroll
                 for (int r = 0; r < 16; ++r) acc[tt][r] *= alpha;
         }
-        if constexpr (!SLOW) {
+        // k-step ks of block tt, the small terms and the hi hi one, of the finite V
+        auto v_at = [&](int tt, int ks, int part) {
+            const half8 v = *(const half8 *)(vp + (2 * ks * HDP + 32 * tt) * 16 + part * kVB);
+            return SLOW && part == 0 ? keep(v, true) : v;
+        };
+        auto pv_lo = [&](floatx16 d, int tt, int ks) {
+            const half8 vh = v_at(tt, ks, 0), vl = v_at(tt, ks, 1);
+            if constexpr (PARTS == 3) {
+                d = mfma32h(v_at(tt, ks, 2), pp[ks][0], d);
+                d = mfma32h(vh, pp[ks][2], d);
+                d = mfma32h(vl, pp[ks][1], d);
+            }
+            d = mfma32h(vl, pp[ks][0], d);
+            return mfma32h(vh, pp[ks][1], d);
+        };
+        auto pv_hi = [&](floatx16 d, int tt, int ks) { return mfma32h(v_at(tt, ks, 0), pp[ks][0], d); };
 #pragma unroll
-            for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-                for (int tt = 0; tt < NT; ++tt) {
-                    const half8 vh = *(const half8 *)(vp + (2 * ks * HDP + 32 * tt) * 16);
-                    const half8 vl = *(const half8 *)(vp + (2 * ks * HDP + 32 * tt) * 16 + kVB);
-                    acc[tt] = mfma32h(vl, ph[ks], acc[tt]);
-                    acc[tt] = mfma32h(vh, pl[ks], acc[tt]);
-                    acc[tt] = mfma32h(vh, ph[ks], acc[tt]);
-                }
+        for (int tt = 0; tt < NT; ++tt) {
+            if constexpr (EXACT) {
+                acc[tt] = pv_hi(pv_lo(acc[tt], tt, 0), tt, 0);
+                acc[tt] = pv_hi(pv_lo(acc[tt], tt, 1), tt, 1);
+            } else {   // the tile's sum, then one rounding at the size of acc
+                acc[tt] += pv_hi(pv_hi(pv_lo(pv_lo(floatx16{}, tt, 0), tt, 1), tt, 0), tt, 1);
+            }
+            if constexpr (SLOW || !EXACT) __builtin_amdgcn_sched_barrier(0);
+        }
+        if constexpr (EXACT && !SLOW) {
             __builtin_amdgcn_sched_group_barrier(kDsRead, 4, 1);
 #pragma unroll
             for (int i = 0; i < 2 * NT - 2; ++i) {
@@ -535,24 +569,17 @@ __global__ __launch_bounds__(kThreads, HDP <= 128 ? 2 : 1) void prefill_kernel(P
                 __builtin_amdgcn_sched_group_barrier(kDsRead, 2, 1);
             }
             __builtin_amdgcn_sched_group_barrier(kMfma, 6, 1);
-        } else {
-            // the finite parts as above; of the non-finite ones, how many +inf,
-            // -inf and NaN every (query, dim) gets from keys it attends (a weight
-            // of 0 for a masked key must not make NaN of them)
+        }
+        if constexpr (SLOW) {
+            // of the non-finite V, how many +inf, -inf and NaN every (query, dim)
+            // gets from keys it attends (a weight of 0 for a masked key must not
+            // make NaN of them)
             half8 on[2];
 #pragma unroll
             for (int r = 0; r < 16; ++r)
                 on[r / 8][r % 8] = k0 + 8 * (r / 4) + 4 * qg + (r % 4) <= qpos ? (_Float16)1.f : (_Float16)0.f;
 #pragma unroll
             for (int tt = 0; tt < NT; ++tt) {
-#pragma unroll
-                for (int ks = 0; ks < 2; ++ks) {
-                    const half8 vh = keep(*(const half8 *)(vp + (2 * ks * HDP + 32 * tt) * 16), true);
-                    const half8 vl = *(const half8 *)(vp + (2 * ks * HDP + 32 * tt) * 16 + kVB);
-                    acc[tt] = mfma32h(vl, ph[ks], acc[tt]);
-                    acc[tt] = mfma32h(vh, pl[ks], acc[tt]);
-                    acc[tt] = mfma32h(vh, ph[ks], acc[tt]);
-                }
                 auto count = [&](auto is, float add) {
                     floatx16 n{};
 #pragma unroll
@@ -578,16 +605,17 @@ __global__ __launch_bounds__(kThreads, HDP <= 128 ? 2 : 1) void prefill_kernel(P
     // tiles after it are then dropped)
     auto run = [&]<bool SLOW>() {
         for (int t = t_begin - 1; t < t_end; ++t) {            // one turn ahead: the first tile's write
-            const int bo = ((t - t_begin) & 1) * kBuf;
+            const int bo = NBUF == 1 ? 0 : ((t - t_begin) & 1) * kBuf;
             if (t >= t_begin) {
                 if constexpr (!SLOW) {
-                    const int4 bv = *(const int4 *)(lds + bo + 2 * kKB + 2 * kVB + 32);
+                    const int4 bv = *(const int4 *)(lds + bo + kMeta + 32);
                     if (__builtin_amdgcn_readfirstlane(bv.x | bv.y | bv.z | bv.w)) return false;   // the same in every wave
                 }
                 compute_tile.template operator()<SLOW>(bo, t);
             }
             if (t + 1 < t_end) {
-                write_tile.template operator()<SLOW>(kBuf - bo);
+                if constexpr (NBUF == 1) __syncthreads();
+                write_tile.template operator()<SLOW>(NBUF == 1 ? 0 : kBuf - bo);
                 if (t + 2 < t_end) load_tile(t + 2);
             }
             __syncthreads();
@@ -639,7 +667,7 @@ __global__ __launch_bounds__(kThreads, HDP <= 128 ? 2 : 1) void prefill_kernel(P
             const int d = 32 * tt + 2 * r + 4 * qg;
             float x[4];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) x[e] = ldexpf(acc[tt][r + e] * inv, sh);
+            for (int e = 0; e < 4; ++e) x[e] = ldexpf(EXACT ? acc[tt][r + e] * inv : acc[tt][r + e] / l_run, sh);
             if (EXACT || d + 4 <= hd) *(f4u *)(dst + d) = f4u{x[0], x[1], x[2], x[3]};
             else if (d + 2 <= hd) *(f2u *)(dst + d) = f2u{x[0], x[1]};
         }
@@ -709,14 +737,21 @@ __global__ __launch_bounds__(256) void prefill_combine_kernel(PrefillArgs a) {
 #pragma unroll
     for (int j = 0; j < N4; ++j) {
         const int d = 32 * j + 4 * c;
-        if (EXACT || d + 4 <= hd) *(f4u *)(op + d) = f4u{acc[j].x * inv, acc[j].y * inv, acc[j].z * inv, acc[j].w * inv};
-        else if (d + 2 <= hd) *(f2u *)(op + d) = f2u{acc[j].x * inv, acc[j].y * inv};
+        const float x[4] = {acc[j].x, acc[j].y, acc[j].z, acc[j].w};
+        float y[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) y[e] = EXACT ? x[e] * inv : x[e] / den;
+        if (EXACT || d + 4 <= hd) *(f4u *)(op + d) = f4u{y[0], y[1], y[2], y[3]};
+        else if (d + 2 <= hd) *(f2u *)(op + d) = f2u{y[0], y[1]};
     }
 }
 
 // ---------------------------------------------------------------- dispatch
 
-int per_cu(int head_dim) { return head_dim <= 128 ? 2 : 1; }   // workgroups that fit a CU
+// head_dim 64 and 128 take the two-part kernel; with a single key tile, where
+// the last bit of V is most of the error, the three-part one (4 keys: 0.9e-7
+// fp32 before, 1.0e-7 two parts)
+bool exact(const PrefillArgs &a) { return (a.hd == 64 || a.hd == 128) && a.pos0 + a.n_tok > kBK; }
 
 template <int HDP, bool EXACT>
 hipError_t launch_t(const PrefillArgs &a, hipStream_t s) {
@@ -743,7 +778,7 @@ void prefill_plan(PrefillArgs &a, int num_cu) {
     a.n_units = 0;
     a.n_kseg = 1;
     a.fold = num_cu;
-    const int cu = per_cu(a.hd), n_wg = a.n_items * a.n_head_kv, F = a.n_tok * a.n_rep;
+    const int cu = per_cu(prefill_padded_dim(a.hd), exact(a)), n_wg = a.n_items * a.n_head_kv, F = a.n_tok * a.n_rep;
     auto tiles = [&](int i) {   // key tiles of item i (its last row)
         const int f0 = kPrefillRows * (a.n_items - 1 - i);
         return (a.pos0 + std::min(f0 + kPrefillRows - 1, F - 1) / a.n_rep) / kBK + 1;
@@ -785,9 +820,9 @@ void prefill_plan(PrefillArgs &a, int num_cu) {
 hipError_t launch_prefill(const PrefillArgs &a, hipStream_t s) {
     switch (prefill_padded_dim(a.hd)) {
         case 32: return launch_t<32, false>(a, s);
-        case 64: return a.hd == 64 ? launch_t<64, true>(a, s) : launch_t<64, false>(a, s);
+        case 64: return exact(a) ? launch_t<64, true>(a, s) : launch_t<64, false>(a, s);
         case 96: return launch_t<96, false>(a, s);
-        case 128: return a.hd == 128 ? launch_t<128, true>(a, s) : launch_t<128, false>(a, s);
+        case 128: return exact(a) ? launch_t<128, true>(a, s) : launch_t<128, false>(a, s);
         case 160: return launch_t<160, false>(a, s);
         case 192: return launch_t<192, false>(a, s);
         case 224: return launch_t<224, false>(a, s);
