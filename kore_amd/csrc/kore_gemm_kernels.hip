@@ -190,8 +190,13 @@ __device__ __forceinline__ int mat_of_tile(const GemmArgs &a, int tile) {
 // First iteration of worker p's run, and the worker whose run holds iteration
 // `it` (the largest p with run_first(p) <= it; runs are never empty because
 // the host keeps workers <= iterations).
-__device__ __forceinline__ int64_t run_first(int64_t T, int P, int p) { return T * p / P; }
-__device__ __forceinline__ int run_of(int64_t T, int P, int64_t it) { return (int)(((it + 1) * P - 1) / T); }
+// Quotients of whole numbers go through doubles, which are exact here: n / d is
+// at least 1 / d below the next whole number, more than 2^-53 of it while n <
+// 2^52, so the rounded quotient never reaches it.  (64-bit integer division is a
+// routine of some 150 instructions, and the fix-up kernels do up to 18 of them.)
+__device__ __forceinline__ int quot(int64_t n, int64_t d) { return (int)((double)n / (double)d); }
+__device__ __forceinline__ int run_first(int64_t T, int P, int p) { return quot(T * p, P); }
+__device__ __forceinline__ int run_of(int64_t T, int P, int64_t it) { return quot((it + 1) * P - 1, T); }
 
 // D block of an MFMA: lane l holds rows 4 (l / 16) + v, activation l % 16 of
 // each 16-block; rows past the matrix and activations past B are dropped.
@@ -271,7 +276,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_kernel(GemmArgs a) {   // tw
     // consecutive runs on one XCD (workgroups are dealt to the 8 XCDs in turn),
     // so the workers that share a split tile share an L2
     const int p = (P % 8 == 0) ? (int)(blockIdx.x % 8) * (P / 8) + (int)(blockIdx.x / 8) : (int)blockIdx.x;
-    const int64_t it0 = run_first(T, P, p), it1 = run_first(T, P, p + 1);
+    const int it0 = run_first(T, P, p), it1 = run_first(T, P, p + 1);
     if (it0 >= it1) return;
     const int64_t cols = (int64_t)nblk * 256;
 
@@ -287,7 +292,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_kernel(GemmArgs a) {   // tw
         return min((tile - a.m[m].tile0) * kGemmRowsPerTile + 16 * wave + i, a.m[m].rows - 1);
     };
 
-    int tile = (int)(it0 / nblk), blk = (int)(it0 % nblk), seg0 = blk;
+    int tile = it0 / nblk, blk = it0 % nblk, seg0 = blk;
     int m = mat_of_tile(a, tile);
     WRaw<Q6> g;
     load_w<Q6>(g, a.m[m], row_of(tile, m), blk, nblk, kk);
@@ -298,7 +303,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_kernel(GemmArgs a) {   // tw
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) acc[nb] = floatx4{0.f, 0.f, 0.f, 0.f};
 
-    for (int64_t it = it0; it < it1; ++it) {
+    for (int it = it0; it < it1; ++it) {
         __syncthreads();                                 // every wave is done with the previous block
 #pragma unroll
         for (int j = 0; j < 4 * NB; ++j) *(floatx4 *)&xs[(wave + 4 * j) * kXStride + 4 * l] = xr[j];
@@ -405,45 +410,15 @@ __global__ __launch_bounds__(kPrepThreads) void gemm16_prep_kernel(const float *
     }
 }
 
-// One lane's weights of one block: Q4_K the header and nibble bytes 64 h ..
-// 64 h + 63; Q6_K ql bytes 64 h .., qh bytes 32 h .., the half's 8 scales, d.
+// One lane's weights of one block (half h of row l % 32): Q4_K the header and
+// nibble bytes 64 h .. 64 h + 63; Q6_K ql bytes 64 h .., qh bytes 32 h .., the
+// half's 8 scales, d.
 template <bool Q6>
 struct W16 {
     uint4 v[Q6 ? 6 : 5];
     uint2 sc;
     uint32_t d;
 };
-
-// Weight loads, non-temporal when nothing reads the same weights again (one
-// unit per tile): the streamed weights then leave the split activations in L2.
-typedef unsigned int u32x4v __attribute__((ext_vector_type(4)));
-typedef unsigned int u32x2v __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ uint4 ld_w4(const uint8_t *p, bool nt) {
-    const u32x4v v = nt ? __builtin_nontemporal_load((const u32x4v *)p) : *(const u32x4v *)p;
-    return make_uint4(v.x, v.y, v.z, v.w);
-}
-__device__ __forceinline__ uint2 ld_w2(const uint8_t *p, bool nt) {
-    const u32x2v v = nt ? __builtin_nontemporal_load((const u32x2v *)p) : *(const u32x2v *)p;
-    return make_uint2(v.x, v.y);
-}
-
-template <bool Q6>
-__device__ __forceinline__ void load_w16(W16<Q6> &g, const GemmMat &m, int row, int blk, int nblk, int h, bool nt) {
-    if (!Q6 || m.type == kQ4K) {
-        const uint8_t *b = m.w + ((int64_t)row * nblk + blk) * kQ4Bytes;
-        g.v[0] = ld_w4(b, nt);
-#pragma unroll
-        for (int k = 0; k < 4; ++k) g.v[1 + k] = ld_w4(b + 16 + 64 * h + 16 * k, nt);
-    } else if constexpr (Q6) {
-        const uint8_t *b = m.w + ((int64_t)row * nblk + blk) * kQ6Body;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) g.v[k] = ld_w4(b + 64 * h + 16 * k, nt);
-        g.v[4] = ld_w4(b + 128 + 32 * h, nt);
-        g.v[5] = ld_w4(b + 128 + 32 * h + 16, nt);
-        g.sc = ld_w2(b + 192 + 8 * h, nt);
-        g.d = m.wd[(int64_t)row * nblk + blk];
-    }
-}
 
 __device__ __forceinline__ uint32_t dword_of(const uint4 *v, int k) {   // dword k of v[0..]
     const uint4 &u = v[k >> 2];
@@ -456,45 +431,77 @@ __device__ __forceinline__ half2v magic2(uint32_t u, uint32_t sel) {
     return __builtin_bit_cast(half2v, __builtin_amdgcn_perm(0x64646464u, u, sel));
 }
 
-// The activations' A operand of k-step s for tile tt, hi and lo parts.
-__device__ __forceinline__ void read_a(const uint8_t *ls, int m, int c, half8 &ahi, half8 &alo) {
-    const int off = m * 512 + ((c ^ (m & 15)) * 16);
-    ahi = *(const half8 *)(ls + off);
-    alo = *(const half8 *)(ls + kG16Lo + off);
-}
-
 __device__ __forceinline__ floatx16 mfma16(half8 a, half8 b, floatx16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
 }
 
-// The A operands (hi, lo) of k-step s for the NT tiles of activations from
-// activation am on (am = 32 for the second half of a halves-mode unit).
+// Half a block's activations in LDS, NA = 32 NT of them: hi [NA][16 chunks],
+// lo the same, 16 bytes a chunk, chunk c of activation m at position c ^ (m &
+// 15) (16 activations' reads hit different banks).  After the second half of a
+// block: the sub-block sums [NA][32 bytes] and 1 / s [NA].
+template <int NT> constexpr int kHalfLo = 32 * NT * 256;
+template <int NT> constexpr int kHalfSx = 2 * kHalfLo<NT>;
+template <int NT> constexpr int kHalfInv = kHalfSx<NT> + 32 * NT * 32;
+template <int NT> constexpr int kHalfEnd = kHalfInv<NT> + 32 * NT * 4;
+
+// The A operands (hi, lo) of k-step s for the NT tiles of activations.
 template <int NT>
-__device__ __forceinline__ void read_step(const uint8_t *ls, int l, int s, int am, half8 (*A)[2]) {
+__device__ __forceinline__ void read_step(const uint8_t *ls, int l, int s, half8 (*A)[2]) {
 #pragma unroll
-    for (int tt = 0; tt < NT; ++tt) read_a(ls, am + 32 * tt + (l & 31), 2 * s + (l >> 5), A[tt][0], A[tt][1]);
+    for (int tt = 0; tt < NT; ++tt) {
+        const int m = 32 * tt + (l & 31), off = m * 256 + (((2 * (s & 7) + (l >> 5)) ^ (m & 15)) * 16);
+        A[tt][0] = *(const half8 *)(ls + off);
+        A[tt][1] = *(const half8 *)(ls + kHalfLo<NT> + off);
+    }
 }
 
-// One Q4_K block: P[tt] = sum_k A x (hi and lo parts); the tiles' MFMA
-// chains alternate.
-template <int NT, bool Q6>
-__device__ __forceinline__ void block16_q4(const W16<Q6> &g, const uint8_t *ls, int l, int am, floatx16 *P) {
+// The instruction order of half a block's 8 k-steps of PER_STEP MFMAs and READS
+// LDS reads each: the reads run LEAD steps ahead of the MFMAs that use them
+// (left alone, the compiler waits for every read right before its MFMA, and a
+// wave spends more time on LDS latency than on MFMAs), and the next step's
+// dequantisation goes between the MFMAs, which run while it issues.
+template <int PER_STEP, int READS, int VALU>
+__device__ __forceinline__ void order_steps() {
+    constexpr int kMfma = 0x8, kValu = 0x2, kDsRead = 0x100, LEAD = 2;
+    __builtin_amdgcn_sched_group_barrier(kDsRead, LEAD * READS, 0);
+    __builtin_amdgcn_sched_group_barrier(kValu, PER_STEP * VALU, 0);
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+#pragma unroll
+        for (int k = 0; k < READS; ++k) {
+            __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(kDsRead, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(kValu, VALU, 0);
+        }
+#pragma unroll
+        for (int k = READS; k < PER_STEP; ++k) {
+            __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(kValu, VALU, 0);
+        }
+    }
+}
+
+// Half HALF of a Q4_K block: P[tt] (+)= sum_k A x (hi and lo parts); the tiles'
+// MFMA chains alternate.
+template <int NT, bool Q6, int HALF>
+__device__ __forceinline__ void block16_q4(const W16<Q6> &g, const uint8_t *ls, int l, floatx16 *P) {
     const int h = l >> 5;
     const uint4 &hdr = g.v[0];
     // scales of sub-blocks 4h .. 4h + 3 as fp16 pairs (sc, sc) and (-1024 sc, -1024 sc)
     half2v scp[4], scn[4];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
+    for (int k = 2 * HALF; k < 2 * HALF + 2; ++k) {
         const _Float16 sc = (_Float16)(float)q4s(hdr, 4 * h + k);
         scp[k] = half2v{sc, sc};
         scn[k] = half2v{(_Float16)(-1024.f) * sc, (_Float16)(-1024.f) * sc};
     }
+    if constexpr (HALF == 0)
 #pragma unroll
-    for (int tt = 0; tt < NT; ++tt) P[tt] = floatx16{};
+        for (int tt = 0; tt < NT; ++tt) P[tt] = floatx16{};
 #pragma unroll
-    for (int s = 0; s < 16; ++s) {
+    for (int s = 8 * HALF; s < 8 * HALF + 8; ++s) {
         half8 A[NT][2];
-        read_step<NT>(ls, l, s, am, A);
+        read_step<NT>(ls, l, s, A);
         const uint32_t D = dword_of(&g.v[1], s);
         const uint32_t L = D & 0x0F0F0F0Fu, H = (D >> 4) & 0x0F0F0F0Fu;
         const int a = s >> 3;                                   // sub-blocks 4h + 2a (low), + 1 (high)
@@ -508,32 +515,34 @@ __device__ __forceinline__ void block16_q4(const W16<Q6> &g, const uint8_t *ls, 
 #pragma unroll
             for (int tt = 0; tt < NT; ++tt) P[tt] = mfma16(A[tt][pp], bw, P[tt]);
     }
+    order_steps<2 * NT, 2 * NT, 10 / NT>();
 }
 
 // Q4_K minimums of one block: M[tt] = sum_j m_j Sx_j, k 0..7 the hi parts of
 // Sx_0..7 times m_0..7, k 8..15 the lo parts times the same.
 template <int NT, bool Q6>
-__device__ __forceinline__ void block16_q4_mins(const W16<Q6> &g, const uint8_t *ls, int l, int am, floatx16 *M) {
+__device__ __forceinline__ void block16_q4_mins(const W16<Q6> &g, const uint8_t *ls, int l, floatx16 *M) {
     const uint4 &hdr = g.v[0];
     half8 bm;
 #pragma unroll
     for (int j = 0; j < 8; ++j) bm[j] = (_Float16)(float)q4m(hdr, j);
 #pragma unroll
     for (int tt = 0; tt < NT; ++tt) {
-        const half8 sx = *(const half8 *)(ls + kG16Sx + (am + 32 * tt + (l & 31)) * 32 + 16 * (l >> 5));
+        const half8 sx = *(const half8 *)(ls + kHalfSx<NT> + (32 * tt + (l & 31)) * 32 + 16 * (l >> 5));
         M[tt] = mfma16(sx, bm, floatx16{});
     }
 }
 
-// One Q6_K block: P[tt] = sum_k (A_hi + A_lo) (x_hi + x_lo) without the lo x lo term.
-template <int NT>
-__device__ __forceinline__ void block16_q6(const W16<true> &g, const uint8_t *ls, int l, int am, floatx16 *P) {
+// Half HALF of a Q6_K block: P[tt] (+)= sum_k (A_hi + A_lo) (x_hi + x_lo) without the lo x lo term.
+template <int NT, int HALF>
+__device__ __forceinline__ void block16_q6(const W16<true> &g, const uint8_t *ls, int l, floatx16 *P) {
+    if constexpr (HALF == 0)
 #pragma unroll
-    for (int tt = 0; tt < NT; ++tt) P[tt] = floatx16{};
+        for (int tt = 0; tt < NT; ++tt) P[tt] = floatx16{};
 #pragma unroll
-    for (int s = 0; s < 16; ++s) {
+    for (int s = 8 * HALF; s < 8 * HALF + 8; ++s) {
         half8 A[NT][2];
-        read_step<NT>(ls, l, s, am, A);
+        read_step<NT>(ls, l, s, A);
         const int a = s >> 3, t = s & 7, sh = 4 * a;
         const uint32_t D1 = dword_of(g.v, t), D2 = dword_of(g.v, 8 + t), Q = dword_of(&g.v[4], t);
         const uint32_t q1 = ((D1 >> sh) & 0x0F0F0F0Fu) | (((Q >> sh) & 0x03030303u) << 4);
@@ -559,6 +568,7 @@ __device__ __forceinline__ void block16_q6(const W16<true> &g, const uint8_t *ls
 #pragma unroll
         for (int tt = 0; tt < NT; ++tt) P[tt] = mfma16(A[tt][0], bl, P[tt]);
     }
+    order_steps<3 * NT, 2 * NT, 12 / NT>();
 }
 
 // D lane l register r of tile tt: activation am + 32 tt + 8 (r / 4) + 4 (l / 32) + r % 4, row l % 32
@@ -583,135 +593,185 @@ __device__ __forceinline__ void store16(const GemmArgs &a, const GemmMat &mt, in
 }
 
 // One workgroup of 8 waves per CU (tiles of 256 rows: each activation block's
-// split is staged once for 256 rows), two LDS buffers: the next block's split
-// activations are copied in (global_load_lds, a linear copy) while the
-// current block's MFMAs run.  The two buffers are separate LDS objects and the
-// loop is unrolled by two, so the compiler sees that reading one does not
-// depend on the copy into the other.  Work units are the tiles, or with
-// a.halves = 2 (NT = 1) each tile's two halves of 32 activations (unit 2 tile
-// + half): twice the units for launches with few tiles, each staging and
-// multiplying half the activations.
+// split is staged once for 256 rows).  Work units are the tiles, or with HV = 2
+// (NT = 1) each tile's two halves of 32 activations (unit 2 tile + half): twice
+// the units for launches with few tiles, each staging and multiplying half the
+// activations.
+//
+// Everything comes in through LDS (global_load_lds).  Activations: a block's two
+// halves (128 columns) have a buffer each, copied in while the other half is
+// multiplied.  Weights: a wave copies the next block of its own 32 rows, in the
+// order of memory, while the current block (taken from LDS into registers
+// before) is multiplied; each 144- or 208-byte block is then one run of
+// consecutive lanes.  Loaded straight to the lanes that use them, 16 bytes of 32
+// rows at a time, every cache line was asked for up to eight times while its
+// first miss was pending, and the waves stood in line for a third of the kernel.
+// What bounds it: the MFMAs (a block takes a CU 4200 cycles of them, 5000 with the
+// dequantisation between, some 7900 with the copies' issue and the two barriers),
+// and a start of 9000 cycles until the first block's data is there, of runs of 4
+// to 5 blocks.  Whole call, pre-pass and fix-up included, against loads straight
+// to registers: 18944 x 3584 Q4_K, 64 activations 39.9 -> 38.4 us; 3584 x 3584
+// 23.0 -> 21.8; 3584 x 18944 Q6_K, 19 activations 42.8 -> 40.9; 8960 x 1536 Q4_K,
+// 22 activations 18.7 -> 17.0.
+// Three LDS objects: the compiler tracks these copies per object, and reading one
+// does not wait for the copies into the others.
 constexpr int kG16Threads = 512;
 
-template <int NT, bool Q6>
+template <int N>
+__device__ __forceinline__ void wait_vm() { __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14)); }
+
+template <int NT, bool Q6, int HV>
 __global__ __launch_bounds__(kG16Threads, 1) void gemm16_kernel(GemmArgs a) {
-    __shared__ __align__(16) uint8_t ls0[kG16BlockBytes];
-    __shared__ __align__(16) uint8_t ls1[kG16BlockBytes];
+    constexpr int NA = 32 * NT;                        // activations of a unit
+    constexpr int kWLoads = Q6 ? 7 : 5;                // 1 KB copies of a wave's weights of a block
+    __shared__ __align__(16) uint8_t ls0[kHalfSx<NT>];
+    __shared__ __align__(16) uint8_t ls1[kHalfEnd<NT>];
+    __shared__ __align__(16) uint8_t lws[8 * kWLoads * 1024];
     const int t = threadIdx.x, l = t & 63;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int h = l >> 5;
-    const int nblk = a.nblk, P = a.workers, hv = a.halves;
-    const int64_t T = (int64_t)a.tiles * hv * nblk;
+    const int nblk = a.nblk, P = a.workers;
+    const int64_t T = (int64_t)a.tiles * HV * nblk;
     const int p = (P % 8 == 0) ? (int)(blockIdx.x % 8) * (P / 8) + (int)(blockIdx.x / 8) : (int)blockIdx.x;
-    const int64_t it0 = run_first(T, P, p), it1 = run_first(T, P, p + 1);
+    const int it0 = run_first(T, P, p), it1 = run_first(T, P, p + 1);
     if (it0 >= it1) return;
-    auto row_of = [&](int tile, int m) {
-        return min((tile - a.m[m].tile0) * kG16Rows + 32 * wave + (l & 31), a.m[m].rows - 1);
+    uint8_t *lw = lws + wave * kWLoads * 1024;
+    auto dma = [&](uint8_t *dst, const uint8_t *src) {
+        __builtin_amdgcn_global_load_lds(src, (void __attribute__((address_space(3))) *)dst, 16, 0, 0);
     };
-    // a block's split activations: 4240 chunks of 16 bytes, copied linearly:
-    // eight rounds of 64 chunks per wave, then the last 144 by waves 0..2
-    constexpr int kChunks = kG16BlockBytes / 16;
-    constexpr int kRounds = kChunks / (8 * 64);
-    static_assert(kG16BlockBytes % 16 == 0 && kChunks - 8 * 64 * kRounds <= 8 * 64, "whole chunks");
-    auto stage = [&](uint8_t *dst, int blk) {
-        const uint8_t *src = a.x16 + (int64_t)blk * kG16BlockBytes + 16 * l;
+    // half H of a block's activations am .. am + NA - 1: 4 activations (256 bytes
+    // of each) per copy of 64 lanes, hi then lo; the sums and 1 / s with the second
+    auto stage = [&](uint8_t *dst, int blk, int am, int H) {
+        const uint8_t *src = a.x16 + (int64_t)blk * kG16BlockBytes + (am + (l >> 4)) * 512 + 256 * H + 16 * (l & 15);
 #pragma unroll
-        for (int k = 0; k < kRounds; ++k) {
-            const int c0 = (k * 8 + wave) * 64;
-            __builtin_amdgcn_global_load_lds(src + 16 * c0, (void __attribute__((address_space(3))) *)(dst + 16 * c0), 16, 0, 0);
+        for (int k = 0; k < NA / 16; ++k) {
+            const int c = 8 * (k % (NA / 32)) + wave;   // group of four activations
+            const int lo = k / (NA / 32);
+            dma(dst + lo * kHalfLo<NT> + c * 1024, src + lo * kG16Lo + c * 2048);
         }
-        const int c0 = (kRounds * 8 + wave) * 64;
-        if (c0 < kChunks && c0 + l < kChunks)
-            __builtin_amdgcn_global_load_lds(src + 16 * c0, (void __attribute__((address_space(3))) *)(dst + 16 * c0), 16, 0, 0);
+        if (H == 0) return;
+        const uint8_t *blkp = a.x16 + (int64_t)blk * kG16BlockBytes;
+        if (wave < NT) dma(dst + kHalfSx<NT> + wave * 1024, blkp + kG16Sx + am * 32 + wave * 1024 + 16 * l);
+        if (wave == NT && l < NA / 4) dma(dst + kHalfInv<NT>, blkp + kG16Inv + am * 4 + 16 * l);
     };
-    // the 32 activations am .. am + 31 of a block (halves mode), at their own
-    // offsets: hi and lo (1024 chunks each, four rounds of 64 per wave), the
-    // sub-block sums (64 chunks, wave 0) and 1 / s (8 chunks, wave 1)
-    auto stage_half = [&](uint8_t *dst, int blk, int am) {
-        const uint8_t *src = a.x16 + (int64_t)blk * kG16BlockBytes + 16 * l;
+    // the wave's 32 rows of a tile (rows past the matrix repeat its last one):
+    // lane offsets of its copies, 16 bytes of row q / chunks each
+    const uint8_t *wbase;
+    const uint16_t *wd = nullptr;
+    uint32_t woff[kWLoads];
+    bool q4 = true;
+    auto set_rows = [&](int tile, int m) {
+        const GemmMat &mt = a.m[m];
+        const int row0 = min((tile - mt.tile0) * kG16Rows + 32 * wave, mt.rows - 1), last = mt.rows - 1 - row0;
+        q4 = !Q6 || mt.type == kQ4K;
+        const int bytes = q4 ? kQ4Bytes : kQ6Body, chunks = bytes / 16;
+        wbase = mt.w + (int64_t)row0 * nblk * bytes;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int c0 = (r < 2 ? 0 : kG16Lo / 16) + am * 32 + 64 * (wave + 8 * (r & 1));
-            __builtin_amdgcn_global_load_lds(src + 16 * c0, (void __attribute__((address_space(3))) *)(dst + 16 * c0), 16, 0, 0);
+        for (int j = 0; j < kWLoads; ++j) {
+            const int q = 64 * j + l, row = q4 ? q / 9 : q / 13, c = q - row * chunks;
+            woff[j] = (uint32_t)min(min(row, 31), last) * (uint32_t)(nblk * bytes) + 16 * c;
         }
-        const int cs = kG16Sx / 16 + am * 2, ci = kG16Inv / 16 + am / 4;
-        if (wave == 0)
-            __builtin_amdgcn_global_load_lds(src + 16 * cs, (void __attribute__((address_space(3))) *)(dst + 16 * cs), 16, 0, 0);
-        if (wave == 1 && l < 8)
-            __builtin_amdgcn_global_load_lds(src + 16 * ci, (void __attribute__((address_space(3))) *)(dst + 16 * ci), 16, 0, 0);
+        if (Q6 && !q4) wd = mt.wd + (int64_t)(row0 + min(l & 31, last)) * nblk;
     };
-    auto stage_unit = [&](uint8_t *dst, int blk, int am) {
-        if (hv == 1) stage(dst, blk);
-        else stage_half(dst, blk, am);
+    // the next block's weights (a Q4_K matrix beside Q6_K ones copies its last
+    // rows again: the count of copies is the same); the Q6_K scale goes to a register
+    auto copy_weights = [&](int blk, uint32_t &d) {
+        const uint8_t *b = wbase + (int64_t)blk * (q4 ? kQ4Bytes : kQ6Body);
+#pragma unroll
+        for (int j = 0; j < kWLoads; ++j) dma(lw + 1024 * j, b + woff[j]);
+        if (Q6 && !q4) d = wd[blk];
+    };
+    auto take_weights = [&](W16<Q6> &g) {
+        if (!Q6 || q4) {
+            const uint8_t *b = lw + (l & 31) * kQ4Bytes;
+            g.v[0] = *(const uint4 *)b;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) g.v[1 + k] = *(const uint4 *)(b + 16 + 64 * h + 16 * k);
+        } else if constexpr (Q6) {
+            const uint8_t *b = lw + (l & 31) * kQ6Body;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) g.v[k] = *(const uint4 *)(b + 64 * h + 16 * k);
+            g.v[4] = *(const uint4 *)(b + 128 + 32 * h);
+            g.v[5] = *(const uint4 *)(b + 128 + 32 * h + 16);
+            g.sc = *(const uint2 *)(b + 192 + 8 * h);
+        }
     };
     // acc += d P - dmin M per block, in the rows' scaled units; times 1 / s of
     // each activation when the tile is stored or left as a partial
-    floatx16 acc[NT];
+    floatx16 acc[NT], Pb[NT];
 #pragma unroll
     for (int tt = 0; tt < NT; ++tt) acc[tt] = floatx16{};
-    auto unscale = [&](const uint8_t *ls, int am) {
+    auto unscale = [&] {
 #pragma unroll
         for (int tt = 0; tt < NT; ++tt)
 #pragma unroll
             for (int qd = 0; qd < 4; ++qd) {
-                const float4 f = *(const float4 *)(ls + kG16Inv + 4 * (am + 32 * tt + 8 * qd + 4 * h));
+                const float4 f = *(const float4 *)(ls1 + kHalfInv<NT> + 4 * (32 * tt + 8 * qd + 4 * h));
                 acc[tt][4 * qd + 0] *= f.x;
                 acc[tt][4 * qd + 1] *= f.y;
                 acc[tt][4 * qd + 2] *= f.z;
                 acc[tt][4 * qd + 3] *= f.w;
             }
     };
-    auto compute = [&](const uint8_t *ls, const W16<Q6> &gc, int cm, int am) {
-        if (Q6 && a.m[cm].type == kQ6K) {
-            floatx16 Pb[NT];
-            if constexpr (Q6) block16_q6<NT>(gc, ls, l, am, Pb);
-            const float d = (float)__builtin_bit_cast(_Float16, (uint16_t)gc.d);
+    auto axpy = [&](float d) {
 #pragma unroll
-            for (int tt = 0; tt < NT; ++tt)
+        for (int tt = 0; tt < NT; ++tt)
 #pragma unroll
-                for (int r = 0; r < 16; ++r) acc[tt][r] = fmaf(d, Pb[tt][r], acc[tt][r]);
-        } else {
-            // d P first, then the minimums in the same registers
-            floatx16 Pb[NT];
-            block16_q4<NT, Q6>(gc, ls, l, am, Pb);
-            const float d = (float)__builtin_bit_cast(_Float16, (uint16_t)(gc.v[0].x & 0xFFFFu));
-            const float dmin = (float)__builtin_bit_cast(_Float16, (uint16_t)(gc.v[0].x >> 16));
-#pragma unroll
-            for (int tt = 0; tt < NT; ++tt)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) acc[tt][r] = fmaf(d, Pb[tt][r], acc[tt][r]);
-            block16_q4_mins<NT, Q6>(gc, ls, l, am, Pb);
-#pragma unroll
-            for (int tt = 0; tt < NT; ++tt)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) acc[tt][r] = fmaf(-dmin, Pb[tt][r], acc[tt][r]);
-        }
+            for (int r = 0; r < 16; ++r) acc[tt][r] = fmaf(d, Pb[tt][r], acc[tt][r]);
     };
 
-    int unit = (int)(it0 / nblk), blk = (int)(it0 % nblk), seg0 = blk;
-    int tile = unit / hv, am = (unit % hv) * 32;
+    int unit = it0 / nblk, blk = it0 % nblk, seg0 = blk;
+    int tile = unit / HV, am = (unit % HV) * 32;
     int m = mat_of_tile(a, tile);
-    W16<Q6> g;
-    load_w16<Q6>(g, a.m[m], row_of(tile, m), blk, nblk, h, hv == 1);
-    stage_unit(ls0, blk, am);
-    __builtin_amdgcn_s_waitcnt(0x0F70);                // vmcnt(0)
+    uint32_t dn = 0;                                   // the copied block's Q6_K scale
+    set_rows(tile, m);
+    copy_weights(blk, dn);
+    stage(ls0, blk, am, 0);
+    wait_vm<0>();
     __syncthreads();
 
-    // one iteration: block `blk` of `unit` from `cur`, the next block's split into `nxt`
-    auto step = [&](int64_t it, const uint8_t *cur, uint8_t *nxt) {
+    // block `blk` of `unit`: its first half and its weights have landed
+    for (int it = it0; it < it1; ++it) {
+        const bool more = it + 1 < it1;
         int nunit = unit, nb = blk + 1;
         if (nb == nblk) { nb = 0; ++nunit; }
-        const int ntile = nunit / hv, nam = (nunit % hv) * 32;
-        const W16<Q6> gc = g;
+        const int ntile = nunit / HV, nam = (nunit % HV) * 32;
         const int cm = m;
-        if (it + 1 < it1) {                            // the next block's activations and weights
-            stage_unit(nxt, nb, nam);
-            m = ntile == tile ? m : mat_of_tile(a, ntile);
-            load_w16<Q6>(g, a.m[m], row_of(ntile, m), nb, nblk, h, hv == 1);
+        const bool cq4 = !Q6 || q4;
+        W16<Q6> g;
+        take_weights(g);
+        if (Q6) g.d = dn;
+        stage(ls1, blk, am, 1);
+        __builtin_amdgcn_s_waitcnt(0xC07F);            // lgkmcnt(0): the weights are out of LDS
+        asm volatile("" ::: "memory");
+        if (more) {
+            if (ntile != tile) {
+                m = mat_of_tile(a, ntile);
+                set_rows(ntile, m);
+            }
+            copy_weights(nb, dn);
         }
-        compute(cur, gc, cm, am);
-        if (it + 1 == it1 || nb == 0) {                // end of this worker's part of the unit
-            unscale(cur, am);
+        if (cq4) {
+            block16_q4<NT, Q6, 0>(g, ls0, l, Pb);
+        } else if constexpr (Q6) {
+            block16_q6<NT, 0>(g, ls0, l, Pb);
+        }
+        if (more) wait_vm<kWLoads>();                  // all but the weights just asked for (or their scale)
+        else wait_vm<0>();
+        __syncthreads();                               // every wave's copies of the second half; ls0 is free
+        if (more) stage(ls0, nb, nam, 0);
+        if (cq4) {
+            // d P first, then the minimums in the same registers
+            block16_q4<NT, Q6, 1>(g, ls1, l, Pb);
+            axpy((float)__builtin_bit_cast(_Float16, (uint16_t)(g.v[0].x & 0xFFFFu)));
+            block16_q4_mins<NT, Q6>(g, ls1, l, Pb);
+            axpy(-(float)__builtin_bit_cast(_Float16, (uint16_t)(g.v[0].x >> 16)));
+        } else if constexpr (Q6) {
+            block16_q6<NT, 1>(g, ls1, l, Pb);
+            axpy((float)__builtin_bit_cast(_Float16, (uint16_t)g.d));
+        }
+        if (!more || nb == 0) {                        // end of this worker's part of the unit
+            unscale();
             if (seg0 != 0 || blk + 1 != nblk) {        // split unit: partial sums for the fix-up launch
                 const int slot = 2 * p + (it0 / nblk == unit ? 0 : 1);
                 float *mine = a.partials + (int64_t)slot * kG16SlotFloats;
@@ -730,13 +790,8 @@ __global__ __launch_bounds__(kG16Threads, 1) void gemm16_kernel(GemmArgs a) {
         tile = ntile;
         am = nam;
         blk = nb;
-        __builtin_amdgcn_s_waitcnt(0x0F70);            // vmcnt(0): the next block's copies have landed
-        __syncthreads();                               // ... for every wave, and `cur` is free
-    };
-    for (int64_t it = it0; it < it1; it += 2) {
-        step(it, ls0, ls1);
-        if (it + 1 >= it1) break;
-        step(it + 1, ls1, ls0);
+        wait_vm<0>();                                  // the next block's first half and weights
+        __syncthreads();                               // ... for every wave, and ls1 is free
     }
 }
 
@@ -999,7 +1054,8 @@ hipError_t launch16_nt(const GemmArgs &a, hipStream_t s) {
                            a.nblk);
         if (hipError_t e = hipGetLastError()) return e;
     }
-    hipLaunchKernelGGL((gemm16_kernel<NT, Q6>), dim3(a.workers), dim3(kG16Threads), 0, s, a);
+    if (NT == 1 && a.halves == 2) hipLaunchKernelGGL((gemm16_kernel<1, Q6, 2>), dim3(a.workers), dim3(kG16Threads), 0, s, a);
+    else hipLaunchKernelGGL((gemm16_kernel<NT, Q6, 1>), dim3(a.workers), dim3(kG16Threads), 0, s, a);
     if (hipError_t e = hipGetLastError()) return e;
     if (a.glu) {   // every gate tile: its SwiGLU is written by the pair's fix-up
         hipLaunchKernelGGL(gemm16_glu_fixup_kernel, dim3(a.m[1].tile0 * a.halves, kG16SlotFloats / 1024),
