@@ -125,10 +125,11 @@ KORE_ATTN_API int kore_attn_prefill_dev(kore_attn_t h, int layer, int pos0, int 
  * No counterpart in kore; it is for callers that cannot allocate (HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  A decode
  * needs n_head x splits x (head_dim + 2) floats, on the MFMA kernels at most
- * 16 x CUs x 130 (532,480 on a 256-CU MI355X), on the generic kernels
- * n_head x head_dim more; a larger need fails with KORE_ATTN_E_UNSUPPORTED.  Every call on one GPU shares the array (each call
- * writes every partial it reads, so nothing carries over): calls that overlap
- * on one GPU (other streams, other handles) race. */
+ * 16 x CUs x 130 (532,480 on a 256-CU MI355X; a larger need fails with
+ * KORE_ATTN_E_UNSUPPORTED); the generic kernels take as many splits as fit.
+ * Every call on one GPU shares the array (each call writes every partial it
+ * reads, so nothing carries over): calls that overlap on one GPU (other
+ * streams, other handles) race. */
 KORE_ATTN_API int kore_attn_decode_noalloc_dev(kore_attn_t h, int layer, int pos, int n_head, int n_head_kv,
                          int head_dim, const float *q, const float *k, const float *v,
                          float *out, void *stream);

@@ -28,8 +28,7 @@ struct kore_attn {
     std::vector<float> inv_freq;
     RopeRow dec_cs{};                        // (cos, sin) of the last decode position
     int dec_cs_pos = -1;
-    float *d_part_o = nullptr;               // decode split partials (o, then max/sum), then
-                                             // the roped q of the generic decode
+    float *d_part_o = nullptr;               // decode split partials (o, then max/sum)
     int max_split = 0;
     size_t part_floats = 0;
     bool fast_decode = false;                // MFMA decode kernels for this geometry
@@ -165,13 +164,15 @@ hipStream_t pick_stream(kore_attn *h, void *stream) {
     return stream ? (hipStream_t)stream : h->stream;
 }
 
-// The decode of a geometry without an MFMA kernel: a prep launch ropes q
-// (into part, after the partials) and appends the new row, then the split
-// attention reads every row up to and including it.
+// The decode of a geometry without an MFMA kernel, in as many splits as part
+// (part_floats floats) holds partials for.
 int generic_decode_enqueue(kore_attn *h, int layer, int pos, const float *q, const float *k, const float *v,
                            float *out, hipStream_t s, float *part, size_t part_floats) {
     const bool wrapped = h->window && pos >= h->window;
     GenericArgs a{};
+    a.q = q;
+    a.k = k;
+    a.v = v;
     a.kc = h->d_k + (size_t)layer * h->layer_floats();
     a.vc = h->d_v + (size_t)layer * h->layer_floats();
     a.out = out;
@@ -179,29 +180,20 @@ int generic_decode_enqueue(kore_attn *h, int layer, int pos, const float *q, con
     a.hd = h->head_dim;
     a.n_head_kv = h->n_head_kv;
     a.n_rep = h->n_head / h->n_head_kv;
-    generic_shape(a.hd, a.n_rep, &a.tile, &a.chunk, &a.n_chunks);
     a.n_rows = wrapped ? h->window : pos + 1;
-    a.rows_per_split = generic_rows_per_split(a.hd, a.n_rep, a.n_rows, a.n_head_kv, h->num_cu);
+    a.new_slot = h->window ? pos % h->window : pos;
+    const size_t hd = (size_t)h->head_dim, fits = part_floats / ((size_t)h->n_head * (hd + 2));
+    a.rows_per_split = generic_rows_per_split(a.n_rows, (int)std::min<size_t>(h->max_split, fits));
     a.n_split = (a.n_rows + a.rows_per_split - 1) / a.rows_per_split;
     a.scale = 1.0f / std::sqrt((float)h->head_dim);   // kore.cpp:1411
-    const size_t np = (size_t)h->n_head * a.n_split, hd = (size_t)h->head_dim;
-    const size_t need = np * (hd + 2) + (size_t)h->n_head * hd;
-    if (need > part_floats)
-        return fail(h, KORE_ATTN_E_UNSUPPORTED, "decode partials need %zu floats, the scratch holds %zu", need,
-                    part_floats);
     a.part_o = part;
-    a.part_ml = part + np * hd;
-    float *q_roped = part + np * (hd + 2);
-    a.q = q_roped;
-    float *kc = h->d_k + (size_t)layer * h->layer_floats(), *vc = h->d_v + (size_t)layer * h->layer_floats();
-    HIP_TRY(h, launch_generic_decode(a, q, k, v, q_roped, kc, vc, h->n_head, h->window ? pos % h->window : pos,
-                                     decode_row(h, pos), s));
+    a.part_ml = part + (size_t)h->n_head * a.n_split * hd;
+    HIP_TRY(h, launch_generic_decode(a, decode_row(h, pos), s));
     return KORE_ATTN_OK;
 }
 
 // Enqueues a decode with its split partials in part (part_floats floats; a
-// decode needs n_head * splits * (head_dim + 2), the generic one n_head *
-// head_dim more).
+// decode needs n_head * splits * (head_dim + 2)).
 int decode_enqueue(kore_attn *h, int layer, int pos, const float *q, const float *k, const float *v,
                    float *out, hipStream_t s, float *part, size_t part_floats) {
     // Cache rows read besides the new one: positions 0..pos-1 (kore.cpp:1437),
@@ -366,12 +358,11 @@ int kore_attn_create(kore_attn_t *out, int n_layer, int ctx, int n_head, int n_h
         release(h);
         return KORE_ATTN_E_HIP;
     }
-    // Decode split partials: n_head * max_split * (hd + 2) floats, and the
-    // roped q of the generic decode.
+    // Decode split partials: n_head * max_split * (hd + 2) floats.
     h->max_split = h->fast_decode ? decode_max_split(head_dim, window ? window : ctx, n_head_kv, h->num_cu)
-                                  : generic_max_split(head_dim, n_rep, n_head_kv, h->num_cu);
+                                  : generic_max_split(n_head_kv, h->num_cu);
     const size_t np = (size_t)n_head * h->max_split;
-    h->part_floats = np * ((size_t)head_dim + 2) + (h->fast_decode ? 0 : (size_t)n_head * head_dim);
+    h->part_floats = np * ((size_t)head_dim + 2);
     if ((e = hipMalloc(&h->d_part_o, h->part_floats * sizeof(float))) != hipSuccess)
         return bail(e, "hipMalloc");
     // Prefill partials of the largest plan: key segments and split halves are

@@ -116,35 +116,31 @@ hipError_t launch_prefill(const PrefillArgs &a, hipStream_t s);
 
 // Decode of any even head_dim up to kMaxGenericHeadDim and any n_rep (the
 // geometries kore accepts, kore.cpp:1278-1290, that the MFMA decode does not
-// cover): tiled attention on VALU with fp64 scores.  A workgroup takes `chunk`
-// q-heads of one kv-head and one split of the cache rows (after a prep launch
-// has roped q and appended the new row).
+// cover): tiled attention on VALU with fp64 scores, a workgroup per kv-head and
+// split of the cache rows, merged by a second launch.
 constexpr int kMaxGenericHeadDim = 2 * kMaxRopeHalf;
 constexpr int kMaxGenericSplits = 128;   // decode splits per kv-head of the generic kernels
+constexpr int kGenTile = 32;             // cache rows per LDS tile
+constexpr int kGenHeads = 8;             // q-heads a workgroup computes at a time
 struct GenericArgs {
-    const float *q;       // roped q [n_head][hd]
-    const float *kc, *vc; // layer base
+    const float *q;       // [n_head][hd]       post-bias, pre-RoPE
+    const float *k;       // [n_head_kv][hd]    post-bias, pre-RoPE
+    const float *v;       // [n_head_kv][hd]
+    float *kc, *vc;       // layer base
     float *out;           // [n_head][hd]
     float *part_o;        // with n_split > 1: [n_head][n_split][hd]
     float *part_ml;       //                   [n_head][n_split][2]
     int slots, hd, n_head_kv, n_rep;
-    int chunk, n_chunks;  // q-heads per workgroup, workgroups per kv-head
-    int tile;             // keys per LDS tile
     int n_rows;           // cache rows attended, [0, n_rows), the new row included
+    int new_slot;         // slot of the new row
     int rows_per_split, n_split;
     float scale;          // kore's 1/sqrt(hd) (kore.cpp:1411)
 };
 bool generic_supported(int head_dim);
-// Launch shape of the generic kernels: tile, chunk and the split bound.
-void generic_shape(int head_dim, int n_rep, int *tile, int *chunk, int *n_chunks);
-int generic_max_split(int head_dim, int n_rep, int n_head_kv, int num_cu);
-int generic_rows_per_split(int head_dim, int n_rep, int n_rows, int n_head_kv, int num_cu);
-size_t generic_lds_bytes(int head_dim, int tile, int chunk);
-// Decode: RoPE of q into q_out and of the new k row, append of k and v at
-// new_slot, then the split attention and (n_split > 1) the merge.
-hipError_t launch_generic_decode(const GenericArgs &a, const float *q, const float *k, const float *v,
-                                 float *q_out, float *kc, float *vc, int n_head, int new_slot, const RopeRow &rr,
-                                 hipStream_t s);
+// Most splits of any decode, and the rows of each for at most max_split of them.
+int generic_max_split(int n_head_kv, int num_cu);
+int generic_rows_per_split(int n_rows, int max_split);
+hipError_t launch_generic_decode(const GenericArgs &a, const RopeRow &rr, hipStream_t s);
 
 // Counter-based synthetic inputs (identical bits to the CPU oracle's
 // generator): dst[r*dim + c] for r < rows.

@@ -17,10 +17,9 @@
 //                          serialises the merge.
 //   append_kernel   RoPE + append of a prefill chunk (kore.cpp:1535-1538).
 //   generic_*       decode of every other geometry kore accepts (any even
-//                   head_dim up to 256, any q-heads per kv-head): a prep launch
-//                   (RoPE of q, RoPE + append of the new row), LDS-tiled
-//                   attention on VALU with fp64 scores for the splits, and the
-//                   merge of their partials.
+//                   head_dim up to 256, any q-heads per kv-head): RoPE, append
+//                   and LDS-tiled attention on VALU with fp64 scores for the
+//                   splits, and the merge of their partials.
 //   synth_kernel    counter-based synthetic inputs for benchmarks and tests.
 //
 // RoPE is bit-exact with kore: cos/sin come from the host-built table (the
@@ -1103,170 +1102,230 @@ __global__ void append_kernel(AppendArgs a, int hd) {
 
 // ------------------------------------------------------------ any geometry
 
-// Block i < n_head: RoPE of q row i at the decode position into q_out; block
-// n_head + g: RoPE of the new k row of kv-head g and the append of k and v at
-// new_slot (kore.cpp:1424-1430).
-__global__ void generic_decode_prep_kernel(const float *q, const float *k, const float *v, float *q_out,
-                                           float *kc, float *vc, int n_head, int hd, int slots, int new_slot,
-                                           RopeRow rr) {
-    const int i = blockIdx.x, half = hd / 2;
-    const bool is_q = i < n_head;
-    const int g = i - n_head;
-    const float *src = is_q ? q + (size_t)i * hd : k + (size_t)g * hd;
-    float *dst = is_q ? q_out + (size_t)i * hd : kc + ((size_t)g * slots + new_slot) * hd;
-    for (int d = threadIdx.x; d < half; d += blockDim.x) {
-        float y0, y1;
-        rope_pair(src[d], src[d + half], make_float2(rr.cs[2 * d], rr.cs[2 * d + 1]), y0, y1);
-        dst[d] = y0;
-        dst[d + half] = y1;
-    }
-    if (!is_q) {
-        float *vd = vc + ((size_t)g * slots + new_slot) * hd;
-        for (int d = threadIdx.x; d < hd; d += blockDim.x) vd[d] = v[(size_t)g * hd + d];
-    }
+// Maximum / sum over the 32 lanes of a half-wave; every one of them receives it.
+__device__ __forceinline__ float max32(float x) {
+    float a, b;
+    pair16(row16_max(x), a, b);
+    return fmaxf(a, b);
+}
+__device__ __forceinline__ float sum32(float x) {
+    x += dpp<0x128>(x);
+    x += dpp<0x124>(x);
+    x += dpp<0x122>(x);
+    x += dpp<0x121>(x);
+    float a, b;
+    pair16(x, a, b);
+    return a + b;
 }
 
-__device__ __forceinline__ double wave_max_d(double x) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) x = fmax(x, __shfl_xor(x, o, 64));
-    return x;
-}
-__device__ __forceinline__ float wave_sum(float x) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
-    return x;
-}
-
-// Workgroup (key range, kv-head g x head chunk c): q-heads g * n_rep + c *
-// chunk + i (i < nh) attend keys [r_begin, r_end) of kv-head g in LDS tiles
-// of `tile` rows (rows past r_end read as zeros, never from memory).  Per
-// tile: scores as fp64 dots of the fp32 roped q and k (each product exact in
-// fp64), times kore's 1/sqrt(hd) and log2(e); one wave per head takes the
-// tile's max and the weights 2^(score - max) with the difference in fp64;
-// then every thread advances its outputs (head, dim) by the weighted V rows
-// in fp32.  Workgroups take split blockIdx.x of the rows [0, n_rows) with q
-// already roped.
-__global__ __launch_bounds__(kThreads) void generic_attend_kernel(GenericArgs a) {
+// Workgroup (split, kv-head g): cache rows [r0, r_end) of kv-head g, the new row
+// (slot new_slot) included, for all q-heads of g, in tiles of kGenTile rows in
+// LDS.  The split that holds the new slot ropes and appends the new row; its
+// cache copy is never read (kore.cpp:1424-1430).
+//
+// A half-wave of 32 lanes is one q-head's: eight heads at a time (more in
+// further passes).  Scores: a lane per row, fp64 dots of the fp32 roped q and k
+// (each product exact), times kore's 1/sqrt(hd) and log2(e); weights 2^(s - m)
+// with the difference in fp64.  Values: a lane per pair of dims, fp32 over the
+// tile's rows in order.  A head's scores, weights and sums stay in its
+// half-wave, so a tile costs two barriers (three where it holds the new row).
+//
+// What bounds it: latency (a launch, the tile's loads, some 2 us of arithmetic;
+// 33/3/96 at 2000 rows: 63 splits of one tile, 189 workgroups).  Before, a launch
+// of its own roped and appended, 8 to 10 heads shared a workgroup of four waves
+// that waited for each other six times a tile, and a thread per output dim walked
+// the splits one load after another in the merge: 33/3/96 at 2000 rows 40 us a
+// layer (5 + 27 + 11, three launches), now 15 (two).
+//
+// VW: floats per load (4 if rows are whole multiples of 16 bytes, else 2).
+template <int VW>
+__global__ __launch_bounds__(kThreads) void generic_decode_kernel(GenericArgs a, RopeRow rr) {
+    typedef float vec __attribute__((ext_vector_type(VW)));
+    constexpr int kBatch = 4;                               // loads in flight per tensor
     extern __shared__ __align__(16) unsigned char g_lds[];
-    const int hd = a.hd, T = a.tile, CH = a.chunk, tid = threadIdx.x;
-    const int lane = tid & 63, wave = tid >> 6;
-    const int g = blockIdx.y / a.n_chunks, c = blockIdx.y % a.n_chunks;
-    const int h0 = c * CH, nh = min(CH, a.n_rep - h0);
-    const int hq0 = g * a.n_rep + h0;
-    const int r_begin = (int)blockIdx.x * a.rows_per_split;
-    const int r_end = min(r_begin + a.rows_per_split, a.n_rows);
-
-    double *s_sc = reinterpret_cast<double *>(g_lds);   // [CH][T] scores
-    float *s_p = reinterpret_cast<float *>(s_sc + CH * T);   // [CH][T] weights
-    float *s_al = s_p + CH * T;                              // [CH] rescale of the tile
-    float *s_m = s_al + CH, *s_l = s_m + CH;                 // [CH] running max, sum
-    float *s_q = s_l + CH;                                   // [CH][hd]
-    float *s_k = s_q + CH * hd;                              // [T][hd + 1]
-    float *s_v = s_k + T * (hd + 1);                         // [T][hd]
-
-    const float *qb = a.q + (size_t)hq0 * hd;
-    for (int e = tid; e < nh * hd; e += kThreads) s_q[e] = qb[e];
-    if (tid < nh) {
-        s_m[tid] = -INFINITY;
-        s_l[tid] = 0.f;
-    }
+    const int hd = a.hd, half = hd / 2, tid = threadIdx.x;
+    const int l32 = tid & 31, slot = tid >> 5;              // head slot of the half-wave
+    const int g = blockIdx.y, split = blockIdx.x;
+    const int r0 = split * a.rows_per_split, r_end = min(r0 + a.rows_per_split, a.n_rows);
+    const int ks = hd + VW;                                 // K row stride: 16-byte reads of 16 rows spread over the banks
+    double *s_q = reinterpret_cast<double *>(g_lds);        // [8][hd]
+    float *s_k = reinterpret_cast<float *>(s_q + kGenHeads * hd);   // [kGenTile][ks]
+    float *s_v = s_k + kGenTile * ks;                       // [kGenTile][hd]
+    float *s_p = s_v + kGenTile * hd;                       // [8][kGenTile]
+    float *kg = a.kc + (size_t)g * a.slots * hd, *vg = a.vc + (size_t)g * a.slots * hd;
     const double sscale = (double)a.scale * 1.4426950408889634;
-    float acc[4] = {0.f, 0.f, 0.f, 0.f};
-    const float *kg = a.kc + (size_t)g * a.slots * hd;
-    const float *vg = a.vc + (size_t)g * a.slots * hd;
-    for (int t0 = r_begin; t0 < r_end; t0 += T) {
-        const int nr = min(T, r_end - t0);
-        __syncthreads();   // the previous tile's readers are done (and s_q, s_m, s_l are set)
-        const float *kt = kg + (size_t)t0 * hd, *vt = vg + (size_t)t0 * hd;
-        for (int e = tid; e < T * hd; e += kThreads) {
-            const int r = e / hd, d = e % hd;
-            const bool ok = r < nr;
-            s_k[r * (hd + 1) + d] = ok ? kt[e] : 0.f;
-            s_v[e] = ok ? vt[e] : 0.f;
+    const int cols = hd / VW, units = kGenTile * cols;
+    const int u_row = tid / cols, u_col = tid - u_row * cols;
+    const int step_row = kThreads / cols, step_col = kThreads - step_row * cols;
+
+    for (int h0 = 0; h0 < a.n_rep; h0 += kGenHeads) {
+        const int nh = min(kGenHeads, a.n_rep - h0);
+        const float *qb = a.q + (size_t)(g * a.n_rep + h0) * hd;
+        if (h0) __syncthreads();                            // the last pass's readers of s_q are done
+        for (int e = tid; e < nh * half; e += kThreads) {
+            const int i = e / half, d = e - i * half;
+            float y0, y1;
+            rope_pair(qb[i * hd + d], qb[i * hd + d + half], make_float2(rr.cs[2 * d], rr.cs[2 * d + 1]), y0, y1);
+            s_q[i * hd + d] = y0;
+            s_q[i * hd + d + half] = y1;
         }
-        __syncthreads();
-        for (int e = tid; e < nh * T; e += kThreads) {
-            const int i = e / T, r = e % T;
-            double s = -INFINITY;
-            if (r < nr) {
-                const float *qi = s_q + i * hd, *kr = s_k + r * (hd + 1);
-                double d0 = 0.0, d1 = 0.0;
-                for (int d = 0; d < hd; d += 2) {
-                    d0 = fma((double)qi[d], (double)kr[d], d0);
-                    d1 = fma((double)qi[d + 1], (double)kr[d + 1], d1);
-                }
-                s = (d0 + d1) * sscale;
-            }
-            s_sc[e] = s;
-        }
-        __syncthreads();
-        for (int i = wave; i < nh; i += kWaves) {
-            const double sv = lane < T ? s_sc[i * T + lane] : -INFINITY;
-            const float m_old = s_m[i];
-            const float m_new = fmaxf(m_old, (float)wave_max_d(sv));
-            const float p = sv != -INFINITY ? fast_exp2((float)(sv - (double)m_new)) : 0.f;
-            const float sum = wave_sum(p);
-            if (lane < T) s_p[i * T + lane] = p;
-            if (lane == 0) {
-                const float al = m_old == -INFINITY ? 0.f : fast_exp2(m_old - m_new);
-                s_al[i] = al;
-                s_m[i] = m_new;
-                s_l[i] = s_l[i] * al + sum;
-            }
-        }
-        __syncthreads();
+        float m_run = -INFINITY, l_run = 0.f;
+        float acc[8];                                       // dims 2 l32 + 64 j + (0, 1)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int o = tid + j * kThreads;
-            if (o < nh * hd) {
-                const int i = o / hd, d = o % hd;
-                const float *pi = s_p + i * T;
-                float x = acc[j] * s_al[i];
-                for (int r = 0; r < nr; ++r) x = fmaf(pi[r], s_v[r * hd + d], x);
-                acc[j] = x;
+        for (int j = 0; j < 8; ++j) acc[j] = 0.f;
+        for (int t0 = r0; t0 < r_end; t0 += kGenTile) {
+            const int nr = min(kGenTile, r_end - t0);
+            if (h0 == 0 || r_end - r0 > kGenTile) {         // a split of one tile keeps it for every pass
+                if (t0 > r0 || h0) __syncthreads();         // the previous tile's readers are done
+                const float *kt = kg + (size_t)t0 * hd, *vt = vg + (size_t)t0 * hd;
+                int row = u_row, col = u_col;
+                for (int e0 = tid; e0 < units; e0 += kBatch * kThreads) {
+                    vec xk[kBatch], xv[kBatch];
+                    int at[kBatch];
+#pragma unroll
+                    for (int u = 0; u < kBatch; ++u) {      // rows past the split read its last one and count as zeros
+                        at[u] = row << 16 | col * VW;
+                        const int o = min(row, nr - 1) * hd + col * VW;
+                        xk[u] = *(const vec *)(kt + o);
+                        xv[u] = *(const vec *)(vt + o);
+                        row += step_row;
+                        col += step_col;
+                        if (col >= cols) {
+                            col -= cols;
+                            ++row;
+                        }
+                    }
+#pragma unroll
+                    for (int u = 0; u < kBatch; ++u) {
+                        const int r = at[u] >> 16, d = at[u] & 0xFFFF;
+                        if (r >= kGenTile) continue;
+                        const bool ok = r < nr;
+#pragma unroll
+                        for (int c = 0; c < VW; ++c) {
+                            xk[u][c] = ok ? xk[u][c] : 0.f;
+                            xv[u][c] = ok ? xv[u][c] : 0.f;
+                        }
+                        *(vec *)(s_k + r * ks + d) = xk[u];
+                        *(vec *)(s_v + r * hd + d) = xv[u];
+                    }
+                }
+                if (a.new_slot >= t0 && a.new_slot < t0 + nr) {
+                    __syncthreads();                        // the stale row is written
+                    const int r = a.new_slot - t0;
+                    const float *kn = a.k + (size_t)g * hd, *vn = a.v + (size_t)g * hd;
+                    for (int d = tid; d < half; d += kThreads) {
+                        float y0, y1;
+                        rope_pair(kn[d], kn[d + half], make_float2(rr.cs[2 * d], rr.cs[2 * d + 1]), y0, y1);
+                        s_k[r * ks + d] = y0;
+                        s_k[r * ks + d + half] = y1;
+                        kg[(size_t)a.new_slot * hd + d] = y0;
+                        kg[(size_t)a.new_slot * hd + d + half] = y1;
+                    }
+                    for (int d = tid; d < hd; d += kThreads) s_v[r * hd + d] = vg[(size_t)a.new_slot * hd + d] = vn[d];
+                }
             }
+            __syncthreads();                                // the tile and s_q are there
+            if (slot >= nh) continue;                       // no barrier is skipped: the loop's are ahead of this
+            // scores: row l32
+            double dot[4] = {0.0, 0.0, 0.0, 0.0};
+            const float *kr = s_k + l32 * ks;
+            const double *qi = s_q + slot * hd;
+#pragma unroll 4
+            for (int d = 0; d < hd; d += VW) {
+                const vec k = *(const vec *)(kr + d);
+#pragma unroll
+                for (int c = 0; c < VW; ++c) dot[c] = fma(qi[d + c], (double)k[c], dot[c]);
+            }
+            const double s = l32 < nr ? ((dot[0] + dot[1]) + (dot[2] + dot[3])) * sscale : -INFINITY;
+            const float m_new = fmaxf(m_run, max32((float)s));
+            const float p = l32 < nr ? fast_exp2((float)(s - (double)m_new)) : 0.f;
+            const float al = m_run == -INFINITY ? 0.f : fast_exp2(m_run - m_new);
+            l_run = l_run * al + sum32(p);
+            m_run = m_new;
+            s_p[slot * kGenTile + l32] = p;
+            __builtin_amdgcn_wave_barrier();                // the half-wave's own weights: LDS keeps a wave's order
+#pragma unroll
+            for (int j = 0; j < 8; ++j) acc[j] *= al;
+            for (int r = 0; r < kGenTile; r += 4) {
+                const float4 p4 = ld4(s_p + slot * kGenTile + r);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const int d = 2 * l32 + 64 * j;
+                    if (d < hd) {
+#pragma unroll
+                        for (int u = 0; u < 4; ++u) {
+                            const float2 v = *(const float2 *)(s_v + (r + u) * hd + d);
+                            acc[2 * j] = fmaf(comp(p4, u), v.x, acc[2 * j]);
+                            acc[2 * j + 1] = fmaf(comp(p4, u), v.y, acc[2 * j + 1]);
+                        }
+                    }
+                }
+            }
+            __builtin_amdgcn_wave_barrier();
         }
+        if (slot < nh) {
+            const int h = g * a.n_rep + h0 + slot;
+            const bool whole = a.n_split == 1;
+            float *dst = whole ? a.out + (size_t)h * hd : a.part_o + ((size_t)h * a.n_split + split) * hd;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int d = 2 * l32 + 64 * j;
+                if (d < hd) {
+                    dst[d] = whole ? acc[2 * j] / l_run : acc[2 * j];
+                    dst[d + 1] = whole ? acc[2 * j + 1] / l_run : acc[2 * j + 1];
+                }
+            }
+            if (!whole && l32 == 0)
+                reinterpret_cast<float2 *>(a.part_ml)[(size_t)h * a.n_split + split] = make_float2(m_run, l_run);
+        }
+    }
+}
+
+// Block h: log-sum-exp merge of q-head h's split partials (at most
+// kMaxGenericSplits; max and sum in the base-2 domain).  Wave w takes splits w,
+// w + 4, ..., eight loads in flight, lane l dims l + 64 j; the waves are summed
+// in LDS.
+__global__ __launch_bounds__(kThreads) void generic_combine_kernel(const float *part_o, const float *part_ml, float *out,
+                                                                   int n_split, int hd) {
+    __shared__ float s_w[kMaxGenericSplits], s_den[kMaxGenericSplits];
+    __shared__ float s_acc[kWaves][kMaxGenericHeadDim];
+    const int h = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const float2 *ml = reinterpret_cast<const float2 *>(part_ml) + (size_t)h * n_split;
+    const float2 m0 = ml[min(lane, n_split - 1)], m1 = ml[min(lane + 64, n_split - 1)];
+    const float m = max4rows(row16_max(fmaxf(m0.x, m1.x)));
+    if (tid < n_split) {
+        const float2 st = tid < 64 ? m0 : m1;
+        const float w = fast_exp2(st.x - m);
+        s_w[tid] = w;
+        s_den[tid] = w * st.y;
     }
     __syncthreads();
-    if (a.n_split == 1) {
+    constexpr int NJ = kMaxGenericHeadDim / 64, kBatch = 8;
+    float acc[NJ];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int o = tid + j * kThreads;
-            if (o < nh * hd) a.out[(size_t)hq0 * hd + o] = acc[j] / s_l[o / hd];
-        }
-    } else {
-        const int sp = blockIdx.x;
+    for (int j = 0; j < NJ; ++j) acc[j] = 0.f;
+    for (int s0 = wave; s0 < n_split; s0 += kWaves * kBatch) {
+        float x[kBatch][NJ];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int o = tid + j * kThreads;
-            if (o < nh * hd) {
-                const int i = o / hd, d = o % hd;
-                a.part_o[((size_t)(hq0 + i) * a.n_split + sp) * hd + d] = acc[j];
+        for (int u = 0; u < kBatch; ++u)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) {
+                const int s = min(s0 + kWaves * u, n_split - 1);
+                x[u][j] = lane + 64 * j < hd ? part_o[((size_t)h * n_split + s) * hd + lane + 64 * j] : 0.f;
             }
-        }
-        if (tid < nh)
-            reinterpret_cast<float2 *>(a.part_ml)[(size_t)(hq0 + tid) * a.n_split + sp] =
-                make_float2(s_m[tid], s_l[tid]);
+#pragma unroll
+        for (int u = 0; u < kBatch; ++u)
+            if (s0 + kWaves * u < n_split)
+#pragma unroll
+                for (int j = 0; j < NJ; ++j) acc[j] = fmaf(s_w[s0 + kWaves * u], x[u][j], acc[j]);
     }
-}
-
-// Block h: log-sum-exp merge of q-head h's split partials (max and sum in
-// the base-2 domain of generic_attend_kernel), one thread per dim.
-__global__ void generic_combine_kernel(const float *part_o, const float *part_ml, float *out, int n_split, int hd) {
-    const int h = blockIdx.x;
-    const float2 *ml = reinterpret_cast<const float2 *>(part_ml) + (size_t)h * n_split;
-    float m = -INFINITY;
-    for (int s = 0; s < n_split; ++s) m = fmaxf(m, ml[s].x);
-    for (int d = threadIdx.x; d < hd; d += blockDim.x) {
-        float acc = 0.f, den = 0.f;
-        for (int s = 0; s < n_split; ++s) {
-            const float2 st = ml[s];
-            const float w = fast_exp2(st.x - m);
-            den = fmaf(w, st.y, den);
-            acc = fmaf(w, part_o[((size_t)h * n_split + s) * hd + d], acc);
-        }
-        out[(size_t)h * hd + d] = acc / den;
-    }
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) s_acc[wave][lane + 64 * j] = acc[j];
+    float den = 0.f;
+    for (int s = 0; s < n_split; ++s) den += s_den[s];
+    __syncthreads();
+    for (int d = tid; d < hd; d += kThreads)
+        out[(size_t)h * hd + d] = ((s_acc[0][d] + s_acc[1][d]) + (s_acc[2][d] + s_acc[3][d])) / den;
 }
 
 // ------------------------------------------------------------------- synth
@@ -1475,47 +1534,37 @@ bool generic_supported(int head_dim) {
     return head_dim >= 2 && head_dim <= kMaxGenericHeadDim && head_dim % 2 == 0;
 }
 
-void generic_shape(int head_dim, int n_rep, int *tile, int *chunk, int *n_chunks) {
-    // K and V tiles within 40 KB; a tile's rows fit one wave (softmax); at
-    // most 1024 (head, dim) outputs (4 per thread) and 1024 (head, row) scores.
-    int T = 64;
-    while (T > 8 && (size_t)T * (2 * head_dim + 1) * sizeof(float) > 40 * 1024) T /= 2;
-    const int ch = std::max(1, std::min({n_rep, 1024 / head_dim, 1024 / T}));
-    *tile = T;
-    *chunk = ch;
-    *n_chunks = (n_rep + ch - 1) / ch;
+int generic_max_split(int n_head_kv, int num_cu) {
+    return std::max(1, std::min(kMaxGenericSplits, 2 * num_cu / std::max(1, n_head_kv)));
 }
 
-size_t generic_lds_bytes(int head_dim, int tile, int chunk) {
-    const size_t T = tile, C = chunk, hd = head_dim;
-    return C * T * sizeof(double) + (C * T + 3 * C + C * hd + T * (hd + 1) + T * hd) * sizeof(float);
+int generic_rows_per_split(int n_rows, int max_split) {
+    // whole tiles (the last split shorter), at most max_split splits: with two
+    // workgroups per CU at most, all of them run at once
+    const int tiles = (n_rows + kGenTile - 1) / kGenTile, S = std::max(1, std::min(max_split, tiles));
+    return std::max(1, (tiles + S - 1) / S) * kGenTile;
 }
 
-int generic_max_split(int head_dim, int n_rep, int n_head_kv, int num_cu) {
-    int T, ch, nc;
-    generic_shape(head_dim, n_rep, &T, &ch, &nc);
-    return std::max(1, std::min(kMaxGenericSplits, num_cu / std::max(1, n_head_kv * nc)));
-}
-
-int generic_rows_per_split(int head_dim, int n_rep, int n_rows, int n_head_kv, int num_cu) {
-    // at most generic_max_split splits, each whole tiles (the last one shorter)
-    int T, ch, nc;
-    generic_shape(head_dim, n_rep, &T, &ch, &nc);
-    const int S = std::max(1, std::min(generic_max_split(head_dim, n_rep, n_head_kv, num_cu), (n_rows + T - 1) / T));
-    const int rps = std::max(1, (n_rows + S - 1) / S);
-    return (rps + T - 1) / T * T;
-}
-
-hipError_t launch_generic_decode(const GenericArgs &a, const float *q, const float *k, const float *v,
-                                 float *q_out, float *kc, float *vc, int n_head, int new_slot, const RopeRow &rr,
-                                 hipStream_t s) {
-    hipLaunchKernelGGL(generic_decode_prep_kernel, dim3(n_head + a.n_head_kv), dim3(64), 0, s, q, k, v, q_out, kc,
-                       vc, n_head, a.hd, a.slots, new_slot, rr);
-    const size_t lds = generic_lds_bytes(a.hd, a.tile, a.chunk);
-    hipLaunchKernelGGL(generic_attend_kernel, dim3(a.n_split, a.n_head_kv * a.n_chunks), dim3(kThreads), lds, s, a);
+hipError_t launch_generic_decode(const GenericArgs &a, const RopeRow &rr, hipStream_t s) {
+    const bool v4 = a.hd % 4 == 0;
+    const int ks = a.hd + (v4 ? 4 : 2);
+    const size_t lds = kGenHeads * (a.hd * sizeof(double) + kGenTile * sizeof(float)) +
+                       (size_t)kGenTile * (ks + a.hd) * sizeof(float);
+    // more than 64 KiB of dynamic LDS (head_dim above 192) needs the kernel's limit raised, once
+    static const hipError_t raised = [] {
+        const int most = 96 * 1024;
+        const hipError_t e = hipFuncSetAttribute((const void *)generic_decode_kernel<4>,
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, most);
+        return e != hipSuccess ? e : hipFuncSetAttribute((const void *)generic_decode_kernel<2>,
+                                                         hipFuncAttributeMaxDynamicSharedMemorySize, most);
+    }();
+    if (raised != hipSuccess) return raised;
+    const dim3 grid(a.n_split, a.n_head_kv);
+    if (v4) hipLaunchKernelGGL(generic_decode_kernel<4>, grid, dim3(kThreads), lds, s, a, rr);
+    else hipLaunchKernelGGL(generic_decode_kernel<2>, grid, dim3(kThreads), lds, s, a, rr);
     if (a.n_split > 1)
-        hipLaunchKernelGGL(generic_combine_kernel, dim3(n_head), dim3(std::min(256, (a.hd + 63) / 64 * 64)), 0, s,
-                           a.part_o, a.part_ml, a.out, a.n_split, a.hd);
+        hipLaunchKernelGGL(generic_combine_kernel, dim3(a.n_head_kv * a.n_rep), dim3(kThreads), 0, s, a.part_o,
+                           a.part_ml, a.out, a.n_split, a.hd);
     return hipGetLastError();
 }
 

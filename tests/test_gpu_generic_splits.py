@@ -1,0 +1,53 @@
+"""The decode of geometries without MFMA kernels at the edges of its tiles: 32-row tiles and splits, the new
+row in every tile position and split, more than eight heads per kv-head (passes), rows of 8- and 16-byte
+multiples, and stale non-finite values in the slot the new row takes.
+
+Reference: the oracle's kore loops; bound 1e-5 of the largest output (fp64 scores; the sums over keys are
+fp32 on both sides, at most 600 of them: 600 * 2^-24 = 3.6e-5 if every rounding went one way, a tenth of it
+as they come)."""
+import numpy as np
+import pytest
+
+import oracle
+
+pytestmark = pytest.mark.gpu
+
+
+def check(nh, nkv, hd, ctx, positions, poison=None):
+    from kore_amd import KoreAttn
+    rng = np.random.default_rng(nh * 1000 + hd + ctx)
+    kv = oracle.KV(1, ctx, nh, nkv, hd, 1e6)
+    n0 = positions[0]
+    with KoreAttn(1, ctx, nh, nkv, hd, 1e6) as a:
+        if n0:
+            x = [rng.standard_normal((n0, h * hd)).astype(np.float32) for h in (nh, nkv, nkv)]
+            a.prefill(0, 0, *x)
+            kv.prefill(0, 0, *x)
+        if poison is not None:   # a row the decode overwrites
+            x = [np.full((1, h * hd), poison, np.float32) for h in (nh, nkv, nkv)]
+            a.prefill(0, n0, *x)
+        for pos in positions:
+            q, k, v = (rng.standard_normal(h * hd).astype(np.float32) for h in (nh, nkv, nkv))
+            out = a.decode(0, pos, q, k, v)
+            ref = kv.decode(0, pos, q, k, v)
+            assert np.max(np.abs(out - ref)) <= 1e-5 * np.max(np.abs(ref)), pos
+        n = positions[-1] + 1
+        kg, vg = a.read_kv(0, 0, n)
+    assert np.array_equal(kg, kv.kcache()[0][:n]) and np.array_equal(vg, kv.vcache()[0][:n])
+
+
+@pytest.mark.parametrize("nh,nkv,hd", [(3, 3, 2), (8, 2, 6), (11, 1, 34), (33, 3, 96), (9, 1, 100), (17, 1, 130),
+                                       (2, 1, 254), (4, 2, 256), (12, 1, 64)])
+@pytest.mark.parametrize("n0", [0, 30, 63, 590])
+def test_edges(nh, nkv, hd, n0):
+    check(nh, nkv, hd, n0 + 4, [n0, n0 + 1, n0 + 2, n0 + 3])
+
+
+@pytest.mark.parametrize("poison", [np.nan, np.inf])
+def test_stale_slot(poison):
+    check(33, 3, 96, 70, [64], poison=poison)
+
+
+def test_many_splits():
+    """More tiles than splits: several tiles each."""
+    check(64, 32, 36, 600, [590, 591])
