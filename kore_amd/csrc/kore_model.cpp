@@ -1,5 +1,6 @@
 // kore_model.cpp - the C ABI of include/kore_model.h: kore's engine_init over a
 // GGUF file with the tensors in HBM, and forward() for one token on the GPU.
+#include "kore_qmv_rows.h"
 #include "kore_model.h"
 
 #include <hip/hip_runtime.h>
@@ -266,9 +267,10 @@ KORE_MODEL_API int kore_model_prefill_dev(kore_model_t m, const int *tokens, int
         if (tokens[z] < 0 || tokens[z] >= m->n_vocab) return fail(m, KORE_MODEL_E_RANGE, "token out of range");
     void *s = stream ? stream : (void *)m->stream;
     const int E = (int)m->hp.n_embd;
-    for (int z = 0; z < n_tok; ++z)                                                       // kore.cpp:1496-1501
-        if (kore_qmv_get_row_dev(m->embd_type, m->embd, tokens[z], E, m->bx + (size_t)z * E, s) != KORE_QMV_OK)
-            return fail(m, KORE_MODEL_E_DEVICE, std::string("embedding: ") + kore_qmv_last_error(nullptr));
+    int64_t rows[64];                                                                     // n_tok <= bsz <= 64
+    for (int z = 0; z < n_tok; ++z) rows[z] = tokens[z];
+    if (kore_qmv_get_rows_dev(m->embd_type, m->embd, rows, n_tok, E, m->bx, s) != KORE_QMV_OK)   // kore.cpp:1496-1501
+        return fail(m, KORE_MODEL_E_DEVICE, std::string("embedding: ") + kore_qmv_last_error(nullptr));
     for (int l = 0; l < (int)m->layers.size(); ++l)
         if (kore_layer_prefill_dev(m->layer, &m->layers[(size_t)l], m->attn, l, pos0, n_tok, m->bx, s) !=
             KORE_LAYER_OK)

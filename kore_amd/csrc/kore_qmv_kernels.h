@@ -97,9 +97,12 @@ hipError_t launch_rmsnorm_rows(const float *x, const float *w, int n, int n_rows
                                uint8_t *x16 = nullptr);
 hipError_t launch_swiglu(float *g, const float *u, int64_t n, hipStream_t s);
 
-// kore's get_row (kore.cpp:384-407): row `row` of a table of rows of n values
-// of type F32 / F16 / BF16 / Q4_K / Q6_K (kore's block bytes) -> out[n] floats.
-hipError_t launch_get_row(int type, const uint8_t *data, int64_t row, int64_t n, float *out, hipStream_t s);
+// kore's get_row (kore.cpp:384-407): rows rows[0 .. n_rows - 1] (at most
+// kMaxGetRows) of a table of rows of n values of type F32 / F16 / BF16 / Q4_K /
+// Q6_K (kore's block bytes) -> out[n_rows][n] floats.
+constexpr int kMaxGetRows = 64;
+hipError_t launch_get_rows(int type, const uint8_t *data, const int64_t *rows, int n_rows, int64_t n, float *out,
+                           hipStream_t s);
 
 // Synthetic GGUF-format weights for benchmarks: nblocks raw Q4_K / Q6_K blocks
 // with hashed bytes and finite f16 scales (dst 2-byte aligned).

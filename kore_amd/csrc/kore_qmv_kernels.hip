@@ -1132,14 +1132,21 @@ namespace {
 
 __device__ __forceinline__ float f16_at(const uint8_t *p) { return f16_bits((uint32_t)p[0] | ((uint32_t)p[1] << 8)); }
 
-// kore's get_row (kore.cpp:384-407): value i of a row of n values, one thread
-// per value.  Q4_K / Q6_K follow kore's dequantisers (kore.cpp:337-381) with
-// their separate roundings (no fused multiply-add).
-__global__ __launch_bounds__(kThreads) void get_row_kernel(int type, const uint8_t *__restrict__ row, int64_t n,
-                                                           float *__restrict__ out) {
+// kore's get_row (kore.cpp:384-407): value i of row blockIdx.y of the list, of n
+// values each, one thread per value.  Q4_K / Q6_K follow kore's dequantisers
+// (kore.cpp:337-381) with their separate roundings (no fused multiply-add).  A
+// chunk's rows are one launch, as a row costs little more than its launch (some 2
+// us): a 1.5B engine of 12 layers, 150 prompt tokens and 8 more 8.28 -> 7.93 ms.
+struct RowList {
+    int64_t row[kMaxGetRows];
+};
+__global__ __launch_bounds__(kThreads) void get_rows_kernel(int type, const uint8_t *__restrict__ data, int64_t row_bytes,
+                                                            int64_t n, float *__restrict__ out, RowList list) {
 #pragma clang fp contract(off)
     const int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
     if (i >= n) return;
+    const uint8_t *row = data + list.row[blockIdx.y] * row_bytes;
+    out += (int64_t)blockIdx.y * n;
     float v = 0.f;
     if (type == 0) {                                     // F32
         v = ((const float *)row)[i];
@@ -1171,16 +1178,21 @@ __global__ __launch_bounds__(kThreads) void get_row_kernel(int type, const uint8
 
 }  // namespace
 
-hipError_t launch_get_row(int type, const uint8_t *data, int64_t row, int64_t n, float *out, hipStream_t s) {
+hipError_t launch_get_rows(int type, const uint8_t *data, const int64_t *rows, int n_rows, int64_t n, float *out,
+                           hipStream_t s) {
     int64_t per = 1, bytes = 4;
     if (type == 1 || type == 30) bytes = 2;
     else if (type == kQ4K) { per = 256; bytes = kQ4Bytes; }
     else if (type == kQ6K) { per = 256; bytes = kQ6Bytes; }
     else if (type != 0) return hipErrorInvalidValue;
-    if (n <= 0 || n % per || row < 0) return hipErrorInvalidValue;
-    const uint8_t *p = data + row * (n / per * bytes);
-    hipLaunchKernelGGL(get_row_kernel, dim3((unsigned)((n + kThreads - 1) / kThreads)), dim3(kThreads), 0, s, type, p,
-                       n, out);
+    if (n <= 0 || n % per || n_rows < 1 || n_rows > kMaxGetRows) return hipErrorInvalidValue;
+    RowList list{};
+    for (int z = 0; z < n_rows; ++z) {
+        if (rows[z] < 0) return hipErrorInvalidValue;
+        list.row[z] = rows[z];
+    }
+    hipLaunchKernelGGL(get_rows_kernel, dim3((unsigned)((n + kThreads - 1) / kThreads), n_rows), dim3(kThreads), 0, s,
+                       type, data, n / per * bytes, n, out, list);
     return hipGetLastError();
 }
 
