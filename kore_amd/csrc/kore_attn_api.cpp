@@ -135,6 +135,22 @@ int ensure_io(kore_attn *h, size_t floats) {
     return KORE_ATTN_OK;
 }
 
+constexpr size_t up4(size_t floats) { return (floats + 3) & ~(size_t)3; }   // whole float4s
+
+// Host rows x[0 .. n - 1] (floats[i] each) one behind the other into the device's
+// staging buffer through the pinned one (up4 of their sum each).  One copy for
+// all: in slices of 256 KiB, to run beside the CPU's own copy, it was slower (a
+// 64-row 7B chunk 137 us a layer against 129, with DMA copies 188).
+int stage_in(kore_attn *h, const float *const *x, const size_t *floats, int n) {
+    size_t at = 0;
+    for (int i = 0; i < n; ++i) {
+        std::memcpy(h->h_stage + at, x[i], floats[i] * sizeof(float));
+        at += floats[i];
+    }
+    HIP_TRY(h, launch_staging(h->h_stage, h->d_io, up4(at), h->stream));
+    return KORE_ATTN_OK;
+}
+
 // Largest number of decode splits any number of cache rows can need.
 int decode_max_split(int head_dim, int max_rows, int n_head_kv, int num_cu) {
     int m = 1;
@@ -402,19 +418,17 @@ int kore_attn_decode(kore_attn_t h, int layer, int pos, int n_head, int n_head_k
     if (int rc = check_decode(h, layer, pos, n_head, n_head_kv, head_dim, q, k, v, out)) return rc;
     HIP_TRY(h, hipSetDevice(h->device));
     const size_t E = (size_t)h->n_head * h->head_dim, kvd = h->kv_dim();
-    if (int rc = ensure_io(h, 2 * E + 2 * kvd)) return rc;
-    float *hs = h->h_stage, *ds = h->d_io;
-    std::memcpy(hs, q, E * sizeof(float));
-    std::memcpy(hs + E, k, kvd * sizeof(float));
-    std::memcpy(hs + E + kvd, v, kvd * sizeof(float));
-    HIP_TRY(h, hipMemcpyAsync(ds, hs, (E + 2 * kvd) * sizeof(float), hipMemcpyHostToDevice, h->stream));
-    if (int rc = decode_enqueue(h, layer, pos, ds, ds + E, ds + E + kvd, ds + E + 2 * kvd, h->stream,
-                                h->d_part_o, h->part_floats))
+    const size_t at = up4(E + 2 * kvd);
+    if (int rc = ensure_io(h, at + up4(E))) return rc;
+    float *ds = h->d_io;
+    const float *x[3] = {q, k, v};
+    const size_t floats[3] = {E, kvd, kvd};
+    if (int rc = stage_in(h, x, floats, 3)) return rc;
+    if (int rc = decode_enqueue(h, layer, pos, ds, ds + E, ds + E + kvd, ds + at, h->stream, h->d_part_o, h->part_floats))
         return rc;
-    HIP_TRY(h, hipMemcpyAsync(hs + E + 2 * kvd, ds + E + 2 * kvd, E * sizeof(float), hipMemcpyDeviceToHost,
-                              h->stream));
+    HIP_TRY(h, launch_staging(ds + at, h->h_stage + at, up4(E), h->stream));
     HIP_TRY(h, hipStreamSynchronize(h->stream));
-    std::memcpy(out, hs + E + 2 * kvd, E * sizeof(float));
+    std::memcpy(out, h->h_stage + at, E * sizeof(float));
     return KORE_ATTN_OK;
 }
 
@@ -457,19 +471,17 @@ int kore_attn_prefill(kore_attn_t h, int layer, int pos0, int n_tok, int n_head,
     if (int rc = check_prefill(h, layer, pos0, n_tok, n_head, n_head_kv, head_dim, q, k, v, out)) return rc;
     HIP_TRY(h, hipSetDevice(h->device));
     const size_t E = (size_t)h->n_head * h->head_dim, kvd = h->kv_dim(), n = (size_t)n_tok;
-    const size_t in_f = n * (E + 2 * kvd);
-    if (int rc = ensure_io(h, in_f + n * E)) return rc;
-    float *hs = h->h_stage, *ds = h->d_io;
-    std::memcpy(hs, q, n * E * sizeof(float));
-    std::memcpy(hs + n * E, k, n * kvd * sizeof(float));
-    std::memcpy(hs + n * (E + kvd), v, n * kvd * sizeof(float));
-    HIP_TRY(h, hipMemcpyAsync(ds, hs, in_f * sizeof(float), hipMemcpyHostToDevice, h->stream));
-    if (int rc = prefill_enqueue(h, layer, pos0, n_tok, ds, ds + n * E, ds + n * (E + kvd), ds + in_f,
-                                 h->stream))
+    const size_t at = up4(n * (E + 2 * kvd));
+    if (int rc = ensure_io(h, at + up4(n * E))) return rc;
+    float *ds = h->d_io;
+    const float *x[3] = {q, k, v};
+    const size_t floats[3] = {n * E, n * kvd, n * kvd};
+    if (int rc = stage_in(h, x, floats, 3)) return rc;
+    if (int rc = prefill_enqueue(h, layer, pos0, n_tok, ds, ds + n * E, ds + n * (E + kvd), ds + at, h->stream))
         return rc;
-    HIP_TRY(h, hipMemcpyAsync(hs + in_f, ds + in_f, n * E * sizeof(float), hipMemcpyDeviceToHost, h->stream));
+    HIP_TRY(h, launch_staging(ds + at, h->h_stage + at, up4(n * E), h->stream));
     HIP_TRY(h, hipStreamSynchronize(h->stream));
-    std::memcpy(out, hs + in_f, n * E * sizeof(float));
+    std::memcpy(out, h->h_stage + at, n * E * sizeof(float));
     return KORE_ATTN_OK;
 }
 

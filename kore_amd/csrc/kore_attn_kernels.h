@@ -142,6 +142,10 @@ int generic_max_split(int n_head_kv, int num_cu);
 int generic_rows_per_split(int n_rows, int max_split);
 hipError_t launch_generic_decode(const GenericArgs &a, const RopeRow &rr, hipStream_t s);
 
+// Copies floats / 4 whole float4s (16-byte aligned) between pinned host memory
+// and the device.
+hipError_t launch_staging(const float *src, float *dst, size_t floats, hipStream_t s);
+
 // Counter-based synthetic inputs (identical bits to the CPU oracle's
 // generator): dst[r*dim + c] for r < rows.
 struct SynthArgs {

@@ -1328,6 +1328,16 @@ __global__ __launch_bounds__(kThreads) void generic_combine_kernel(const float *
         out[(size_t)h * hd + d] = ((s_acc[0][d] + s_acc[1][d]) + (s_acc[2][d] + s_acc[3][d])) / den;
 }
 
+// ------------------------------------------------------------------ staging
+
+// n4 float4s between pinned host memory and the device, either way.  Bound by
+// the bus (1.1 MiB in some 22 us); the DMA engine takes as long and hands over to
+// and from the kernels beside it, which this one, on the kernels' own queue, does
+// not: a 64-row 7B chunk from host buffers 134 -> 129 us a layer.
+__global__ __launch_bounds__(kThreads) void staging_kernel(const float4 *__restrict__ src, float4 *__restrict__ dst, size_t n4) {
+    for (size_t i = blockIdx.x * (size_t)kThreads + threadIdx.x; i < n4; i += (size_t)gridDim.x * kThreads) dst[i] = src[i];
+}
+
 // ------------------------------------------------------------------- synth
 
 __device__ __forceinline__ uint64_t splitmix64(uint64_t x) {
@@ -1565,6 +1575,14 @@ hipError_t launch_generic_decode(const GenericArgs &a, const RopeRow &rr, hipStr
     if (a.n_split > 1)
         hipLaunchKernelGGL(generic_combine_kernel, dim3(a.n_head_kv * a.n_rep), dim3(kThreads), 0, s, a.part_o,
                            a.part_ml, a.out, a.n_split, a.hd);
+    return hipGetLastError();
+}
+
+hipError_t launch_staging(const float *src, float *dst, size_t floats, hipStream_t s) {
+    const size_t n4 = floats / 4;
+    if (n4 == 0) return hipSuccess;
+    hipLaunchKernelGGL(staging_kernel, dim3((unsigned)std::min<size_t>(512, (n4 + kThreads - 1) / kThreads)), dim3(kThreads),
+                       0, s, reinterpret_cast<const float4 *>(src), reinterpret_cast<float4 *>(dst), n4);
     return hipGetLastError();
 }
 
