@@ -374,6 +374,7 @@ int kore_attn_create(kore_attn_t *out, int n_layer, int ctx, int n_head, int n_h
         release(h);
         return KORE_ATTN_E_HIP;
     }
+    if (!h->fast_decode && (e = prepare_generic_decode(head_dim)) != hipSuccess) return bail(e, "hipFuncSetAttribute");
     // Decode split partials: n_head * max_split * (hd + 2) floats.
     h->max_split = h->fast_decode ? decode_max_split(head_dim, window ? window : ctx, n_head_kv, h->num_cu)
                                   : generic_max_split(n_head_kv, h->num_cu);

@@ -1555,20 +1555,21 @@ int generic_rows_per_split(int n_rows, int max_split) {
     return std::max(1, (tiles + S - 1) / S) * kGenTile;
 }
 
+static size_t generic_lds_bytes(int hd) {
+    const int ks = hd + (hd % 4 == 0 ? 4 : 2);
+    return kGenHeads * (hd * sizeof(double) + kGenTile * sizeof(float)) + (size_t)kGenTile * (ks + hd) * sizeof(float);
+}
+
+hipError_t prepare_generic_decode(int head_dim) {
+    const int lds = (int)generic_lds_bytes(head_dim);
+    const void *f = head_dim % 4 == 0 ? (const void *)generic_decode_kernel<4> : (const void *)generic_decode_kernel<2>;
+    if (lds <= 64 * 1024) return hipSuccess;
+    return hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)generic_lds_bytes(kMaxGenericHeadDim));
+}
+
 hipError_t launch_generic_decode(const GenericArgs &a, const RopeRow &rr, hipStream_t s) {
     const bool v4 = a.hd % 4 == 0;
-    const int ks = a.hd + (v4 ? 4 : 2);
-    const size_t lds = kGenHeads * (a.hd * sizeof(double) + kGenTile * sizeof(float)) +
-                       (size_t)kGenTile * (ks + a.hd) * sizeof(float);
-    // more than 64 KiB of dynamic LDS (head_dim above 192) needs the kernel's limit raised, once
-    static const hipError_t raised = [] {
-        const int most = 96 * 1024;
-        const hipError_t e = hipFuncSetAttribute((const void *)generic_decode_kernel<4>,
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize, most);
-        return e != hipSuccess ? e : hipFuncSetAttribute((const void *)generic_decode_kernel<2>,
-                                                         hipFuncAttributeMaxDynamicSharedMemorySize, most);
-    }();
-    if (raised != hipSuccess) return raised;
+    const size_t lds = generic_lds_bytes(a.hd);
     const dim3 grid(a.n_split, a.n_head_kv);
     if (v4) hipLaunchKernelGGL(generic_decode_kernel<4>, grid, dim3(kThreads), lds, s, a, rr);
     else hipLaunchKernelGGL(generic_decode_kernel<2>, grid, dim3(kThreads), lds, s, a, rr);
