@@ -477,7 +477,11 @@ __global__ __launch_bounds__(kThreads, per_cu(HDP, EXACT)) void prefill_kernel(P
         }
         // s[r]: query qi, key k0 + 8 (r / 4) + 4 qg + r % 4; the causal mask only
         // matters on tiles that reach past the strip's first row
-        const float cj[4] = {cq * ck.x, cq * ck.y, cq * ck.z, cq * ck.w};
+        // (never 0, which an operand of zeros or of tiny values would make it: a
+        // masked score of -inf times 0 is NaN)
+        constexpr float kTiny = 0x1p-126f;
+        const float cj[4] = {fmaxf(cq * ck.x, kTiny), fmaxf(cq * ck.y, kTiny), fmaxf(cq * ck.z, kTiny),
+                             fmaxf(cq * ck.w, kTiny)};
         const bool diag = k0 + kBK - 1 > my_kmin;
         float mt = -INFINITY;
         if (diag) {
