@@ -1238,7 +1238,8 @@ __global__ __launch_bounds__(kThreads) void generic_decode_kernel(GenericArgs a,
             }
             const double s = l32 < nr ? ((dot[0] + dot[1]) + (dot[2] + dot[3])) * sscale : -INFINITY;
             const float m_new = fmaxf(m_run, max32((float)s));
-            const float p = l32 < nr ? fast_exp2((float)(s - (double)m_new)) : 0.f;
+            // a score of -inf weighs nothing, also where every row so far has it
+            const float p = s != -INFINITY ? fast_exp2((float)(s - (double)m_new)) : 0.f;
             const float al = m_run == -INFINITY ? 0.f : fast_exp2(m_run - m_new);
             l_run = l_run * al + sum32(p);
             m_run = m_new;

@@ -51,3 +51,26 @@ def test_stale_slot(poison):
 def test_many_splits():
     """More tiles than splits: several tiles each."""
     check(64, 32, 36, 600, [590, 591])
+
+
+@pytest.mark.parametrize("nh,nkv,hd,n0,bad", [(33, 3, 96, 32, range(32, 33)),     # the new row, alone in its tile and split
+                                              (2, 2, 34, 64, range(64, 65)),
+                                              (64, 32, 36, 598, range(64, 96)),   # the first of a split's two tiles
+                                              (64, 32, 36, 598, range(96, 128)),  # the second
+                                              (64, 32, 36, 598, range(64, 128))]) # a whole split
+def test_tile_of_minus_infinity(nh, nkv, hd, n0, bad):
+    """Rows whose scores are -inf (an infinity in K against a q of the other sign) weigh nothing, also where they
+    are all of a tile."""
+    from kore_amd import KoreAttn
+    rng = np.random.default_rng(5)
+    q, k, v = (rng.standard_normal((n0 + 1, h * hd)).astype(np.float32) for h in (nh, nkv, nkv))
+    for d in (hd // 2 - 1, hd - 1):                  # the pair with the slowest rotation: both stay below 0
+        q[:, d::hd] = -1.0
+    k.reshape(-1, nkv, hd)[list(bad), :, hd // 2 - 1] = np.inf
+    kv = oracle.KV(1, n0 + 1, nh, nkv, hd, 1e6)
+    with KoreAttn(1, n0 + 1, nh, nkv, hd, 1e6) as a, np.errstate(invalid="ignore"):
+        a.prefill(0, 0, q[:n0], k[:n0], v[:n0])
+        kv.prefill(0, 0, q[:n0], k[:n0], v[:n0])
+        out, ref = a.decode(0, n0, q[n0], k[n0], v[n0]), kv.decode(0, n0, q[n0], k[n0], v[n0])
+    assert np.all(np.isfinite(ref))
+    assert np.max(np.abs(out - ref)) <= 1e-5 * np.max(np.abs(ref))
