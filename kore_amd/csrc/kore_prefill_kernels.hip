@@ -32,7 +32,8 @@
 // by its own, K and V by groups of eight keys, a query's softmax weights by one
 // that follows them.  A value's parts go down to 2^-25, so what a small one loses
 // is 2^-38 of its group's largest.  Where that could be seen in an output (V
-// whose keys, dims, groups or tiles lie far apart in size) or a value is
+// whose keys, dims, groups or tiles lie far apart in size, or K and q that make
+// a score coarse) or a value is
 // not finite, the workgroup starts again on prefill_fp32, as the fp32 products
 // were (2.5 times the time of this kernel): such values reach exactly the rows
 // that attend them.
@@ -806,7 +807,13 @@ __global__ __launch_bounds__(kThreads, per_cu(HDP, EXACT)) void prefill_kernel(P
         bool move = z > kTMax;
         if constexpr (EXACT) move |= z < t_min;
         else move |= (alpha != 1.f) | (!settled && z < kTMin);
-        if (__builtin_amdgcn_ballot_w64(move)) {
+        // Small elements of q and K are off by 2^-25, scaled, beside partners of up to
+        // 2^14: a score by some 2^-7 times its factor.  That has to be below 2^-21 (3e-7
+        // of a weight), or below what fp32 leaves of a score as large as the tile's
+        // largest (a channel that is large in q and in K).
+        const float cm = fmaxf(fmaxf(cj[0], cj[1]), fmaxf(cj[2], cj[3]));
+        if (__builtin_amdgcn_ballot_w64(move | (cm > 0x1p-14f))) {
+            off |= __builtin_amdgcn_ballot_w64(cm > 0x1p-15f * __builtin_fabsf(mt) && cm > 0x1p-14f) != 0;
             move &= mt != -INFINITY;
             if (__builtin_amdgcn_ballot_w64(move)) {
                 float am = 0.f, lo, hi;

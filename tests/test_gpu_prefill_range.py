@@ -128,7 +128,8 @@ def test_zero_v_of_some_keys(nh, nkv, hd):
     k[zero, ::hd] = 2.0 * np.float32(np.sqrt(hd))
     q, k = unrotate(q, np.arange(70, 110), hd), unrotate(k, np.arange(110), hd)
     v[zero] = 0.0
-    check(q, k, v, 70, nh, nkv, hd, tol=4e-6)         # arguments of up to 16 * 1.45
+    # scores of 16 and their differences, in base 2, each rounded in fp32
+    check(q, k, v, 70, nh, nkv, hd, tol=1e-6 + 16 * 1.45 * 2.0 ** -22 * 0.69)
 
 
 @pytest.mark.parametrize("nh,nkv,hd,n,pos0", [(7, 1, 128, 300, 500),      # key segments
@@ -146,3 +147,36 @@ def test_large_v_where_the_work_is_split(nh, nkv, hd, n, pos0, key):
             ref = reference(q[z:z + 1], k[:p + 1], v[:p + 1], p, nh, nkv, hd)[0]
             err = np.linalg.norm(out[z] - ref, axis=-1) / np.linalg.norm(ref, axis=-1)
             assert err.max() <= 1e-6, (z, err.max())
+
+
+@pytest.mark.parametrize("nh,nkv,hd", GEOMETRIES)
+@pytest.mark.parametrize("f", [1e2, 1e3, 1e4, 1e6, 1e8, 1e16, 1e30])
+def test_large_k_of_a_later_key(nh, nkv, hd, f):
+    """K of position 60 is f times its neighbours' in its group: rows before it do not attend it."""
+    q, k, v = inputs(64, 0, nh, nkv, hd, 17)
+    k[60] *= np.float32(f)
+    check(q, k, v, 0, nh, nkv, hd, rows=slice(0, 60))
+
+
+@pytest.mark.parametrize("nh,nkv,hd", GEOMETRIES)
+@pytest.mark.parametrize("f", [1e4, 1e8])
+def test_large_k_of_a_negligible_key(nh, nkv, hd, f):
+    """Position 61's K is f times the others' and its score far below theirs."""
+    q, k, v = inputs(60, 70, nh, nkv, hd, 18)
+    q[:, ::hd] = 3.0
+    k[:, ::hd] = 0.5
+    k[61, ::hd] = -np.float32(f) * 30
+    k[61].reshape(nkv, hd)[:, 1:] = 0.0
+    q, k = unrotate(q, np.arange(70, 130), hd), unrotate(k, np.arange(130), hd)
+    check(q, k, v, 70, nh, nkv, hd)
+
+
+@pytest.mark.parametrize("nh,nkv,hd", GEOMETRIES)
+def test_large_channel_of_q_that_k_lacks(nh, nkv, hd):
+    """q's largest channel is 1e7 times the others, and every K is zero there."""
+    q, k, v = inputs(40, 40, nh, nkv, hd, 19)
+    q[:, ::hd] = 1e7
+    q[:, hd // 2::hd] = 0.0
+    k[:, ::hd] = 0.0
+    k[:, hd // 2::hd] = 0.0
+    check(q, k, v, 40, nh, nkv, hd)
