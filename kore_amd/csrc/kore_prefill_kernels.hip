@@ -693,6 +693,7 @@ __global__ __launch_bounds__(kThreads, per_cu(HDP, EXACT)) void prefill_kernel(P
     float base = -INFINITY, t_min = kTMin;         // EXACT: m_run - unit; kTMin while acc is below kEnough, else -inf
     bool settled = false;                          // not EXACT: every query's acc is above kEnough
     int a_min = kZeroExp, a_max = -kZeroExp;       // V's scales so far
+    bool begun = false;                            // acc is no longer zero
 
     auto compute_tile = [&](int bo, int t) {
         const int k0 = t * kBK;
@@ -816,13 +817,16 @@ __global__ __launch_bounds__(kThreads, per_cu(HDP, EXACT)) void prefill_kernel(P
             off |= __builtin_amdgcn_ballot_w64(cm > 0x1p-15f * __builtin_fabsf(mt) && cm > 0x1p-14f) != 0;
             move &= mt != -INFINITY;
             if (__builtin_amdgcn_ballot_w64(move)) {
-                float am = 0.f, lo, hi;
+                float am = 0.f;
+                if (begun) {
+                    float lo, hi;
 #pragma unroll
-                for (int tt = 0; tt < NT; ++tt)
+                    for (int tt = 0; tt < NT; ++tt)
 #pragma unroll
-                    for (int r = 0; r < 16; ++r) am = fmaxf(am, __builtin_fabsf(acc[tt][r]));
-                pair32(am, lo, hi);
-                am = fmaxf(lo, hi);
+                        for (int r = 0; r < 16; ++r) am = fmaxf(am, __builtin_fabsf(acc[tt][r]));
+                    pair32(am, lo, hi);
+                    am = fmaxf(lo, hi);
+                }
                 const bool first = EXACT ? base == -INFINITY : unit == kNone;
                 if constexpr (EXACT) {
                     const float m_new = move && (first || mt > m_run) ? ceilf(mt) : m_run;
@@ -843,12 +847,14 @@ __global__ __launch_bounds__(kThreads, per_cu(HDP, EXACT)) void prefill_kernel(P
                 } else {
                     settled = __builtin_amdgcn_ballot_w64(am < kEnough) == 0;
                 }
+                if (begun)
 #pragma unroll
-                for (int tt = 0; tt < NT; ++tt)
+                    for (int tt = 0; tt < NT; ++tt)
 #pragma unroll
-                    for (int r = 0; r < 16; ++r) acc[tt][r] *= alpha;
+                        for (int r = 0; r < 16; ++r) acc[tt][r] *= alpha;
             }
         }
+        begun = true;
         if constexpr (EXACT) {
             const float ps = weights(m_run);
             l_run += ps;
