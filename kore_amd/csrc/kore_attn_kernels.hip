@@ -75,13 +75,6 @@ __device__ unsigned long long g_tl_comb[kTlComb * kTlCombStamps];
 
 // ------------------------------------------------------------------ decode
 
-// The decode kernels start at a page.  Inside a layer they run between other
-// kernels, their code is fetched anew each time, and where the linker puts them
-// (wherever the kernels before them end) decides how many pages that touches:
-// four 7B layers of a decode step 250.0 us with the combine across a page boundary
-// and the split's first 256 bytes on a page of their own, 246.7 aligned.
-#define KERNEL_PAGE __attribute__((aligned(4096)))
-
 // v_mfma_f32_16x16x4f32, one block: lane l supplies A[l%16][l/16] and
 // B[l/16][l%16]; D register v of lane l is D[4(l/16) + v][l%16].
 __device__ __forceinline__ floatx4 mfma16(float a, float b, floatx4 c) {
@@ -182,7 +175,6 @@ __device__ __forceinline__ double sum4rows_d(double x) {
 // the build with the whole register file (280 there): 7B at 4096 rows 8.14-
 // 8.20 against 8.32-8.34 us per layer.
 template <int HD, int NR>
-KERNEL_PAGE
 __global__ __launch_bounds__(kThreads, 2) void decode_split_kernel(const float *__restrict__ q_in, float *kc_in,
                                                                 float *vc_in, const float *__restrict__ k_in,
                                                                 const float *__restrict__ v_in, int n_rows,
@@ -605,7 +597,6 @@ __global__ __launch_bounds__(kThreads, 2) void decode_split_kernel(const float *
 // states and one row per wave measured 0.4-0.8 us slower here (a loop that
 // streams at the read rate, and a different register allocation).
 template <int HD, int NR>
-KERNEL_PAGE
 __global__ __launch_bounds__(kThreads) void decode_multi_kernel(const float *__restrict__ q_in, float *kc_in,
                                                                 float *vc_in, const float *__restrict__ k_in,
                                                                 const float *__restrict__ v_in, int n_rows,
@@ -1035,7 +1026,6 @@ __global__ __launch_bounds__(kThreads) void decode_multi_kernel(const float *__r
 // chunk is one whole 128-byte line; every load is issued before the first
 // use (one memory round trip).
 template <int HD, int PER>
-KERNEL_PAGE
 __global__ __launch_bounds__(64) void decode_combine_kernel(const float *part_o, const float *part_ml, float *out,
                                                             int n_split) {
     TL_DECL(kTlCombStamps);
