@@ -1135,7 +1135,8 @@ __device__ __forceinline__ float sum32(float x) {
 // of its own roped and appended, 8 to 10 heads shared a workgroup of four waves
 // that waited for each other six times a tile, and a thread per output dim walked
 // the splits one load after another in the merge: 33/3/96 at 2000 rows 40 us a
-// layer (5 + 27 + 11, three launches), now 15 (two).
+// layer (5 + 27 + 11, three launches), now 15 (two), at 2.4e-7 of the 2-norm from
+// float64 (2.8e-7 before).
 //
 // VW: floats per load (4 if rows are whole multiples of 16 bytes, else 2).
 template <int VW>
@@ -1237,7 +1238,8 @@ __global__ __launch_bounds__(kThreads) void generic_decode_kernel(GenericArgs a,
                 for (int c = 0; c < VW; ++c) dot[c] = fma(qi[d + c], (double)k[c], dot[c]);
             }
             const double s = l32 < nr ? ((dot[0] + dot[1]) + (dot[2] + dot[3])) * sscale : -INFINITY;
-            const float m_new = fmaxf(m_run, max32((float)s));
+            // an integer above the maximum as reference: al, and the merge's factors, are exact
+            const float m_new = fmaxf(m_run, ceilf(max32((float)s)));
             // a score of -inf weighs nothing, also where every row so far has it
             const float p = s != -INFINITY ? fast_exp2((float)(s - (double)m_new)) : 0.f;
             const float al = m_run == -INFINITY ? 0.f : fast_exp2(m_run - m_new);
@@ -1288,18 +1290,20 @@ __global__ __launch_bounds__(kThreads) void generic_decode_kernel(GenericArgs a,
 // in LDS.
 __global__ __launch_bounds__(kThreads) void generic_combine_kernel(const float *part_o, const float *part_ml, float *out,
                                                                    int n_split, int hd) {
-    __shared__ float s_w[kMaxGenericSplits], s_den[kMaxGenericSplits];
+    __shared__ float s_w[kMaxGenericSplits];
     __shared__ float s_acc[kWaves][kMaxGenericHeadDim];
     const int h = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const float2 *ml = reinterpret_cast<const float2 *>(part_ml) + (size_t)h * n_split;
     const float2 m0 = ml[min(lane, n_split - 1)], m1 = ml[min(lane + 64, n_split - 1)];
     const float m = max4rows(row16_max(fmaxf(m0.x, m1.x)));
-    if (tid < n_split) {
-        const float2 st = tid < 64 ? m0 : m1;
-        const float w = fast_exp2(st.x - m);
-        s_w[tid] = w;
-        s_den[tid] = w * st.y;
+    const float w0 = lane < n_split ? fast_exp2(m0.x - m) : 0.f, w1 = lane + 64 < n_split ? fast_exp2(m1.x - m) : 0.f;
+    if (wave == 0) {
+        s_w[lane] = w0;
+        s_w[lane + 64] = w1;
     }
+    float d0, d1;
+    pair32(sum32(fmaf(w0, m0.y, w1 * m1.y)), d0, d1);
+    const float den = d0 + d1;
     __syncthreads();
     constexpr int NJ = kMaxGenericHeadDim / 64, kBatch = 8;
     float acc[NJ];
@@ -1322,8 +1326,6 @@ __global__ __launch_bounds__(kThreads) void generic_combine_kernel(const float *
     }
 #pragma unroll
     for (int j = 0; j < NJ; ++j) s_acc[wave][lane + 64 * j] = acc[j];
-    float den = 0.f;
-    for (int s = 0; s < n_split; ++s) den += s_den[s];
     __syncthreads();
     for (int d = tid; d < hd; d += kThreads)
         out[(size_t)h * hd + d] = ((s_acc[0][d] + s_acc[1][d]) + (s_acc[2][d] + s_acc[3][d])) / den;

@@ -74,3 +74,22 @@ def test_tile_of_minus_infinity(nh, nkv, hd, n0, bad):
         out, ref = a.decode(0, n0, q[n0], k[n0], v[n0]), kv.decode(0, n0, q[n0], k[n0], v[n0])
     assert np.all(np.isfinite(ref))
     assert np.max(np.abs(out - ref)) <= 1e-5 * np.max(np.abs(ref))
+
+
+def test_many_rows_against_float64():
+    """63 splits merged.  2-norm of the error, mean of six draws: 1.56e-7, and 1.98e-7 where the sum of the weights
+    is added up one split after the other and the factors between splits are rounded."""
+    from kore_amd import KoreAttn
+    from tests.test_gpu_prefill_split import reference
+    nh, nkv, hd, n0, errs = 33, 3, 96, 2000, []
+    for seed in range(6):
+        rng = np.random.default_rng(seed)
+        q, k, v = (rng.standard_normal((n0 + 1, h * hd)).astype(np.float32) for h in (nh, nkv, nkv))
+        q[:, ::17] *= 4
+        k[:, ::17] *= 4
+        with KoreAttn(1, n0 + 1, nh, nkv, hd, 1e4) as a:
+            a.prefill(0, 0, np.zeros_like(q[:n0]), k[:n0], v[:n0])
+            out = a.decode(0, n0, q[n0], k[n0], v[n0]).reshape(nh, hd)
+        ref = reference(q[n0:], k, v, n0, nh, nkv, hd)[0]
+        errs.append(np.linalg.norm(out - ref) / np.linalg.norm(ref))
+    assert np.mean(errs) <= 1.8e-7, errs
