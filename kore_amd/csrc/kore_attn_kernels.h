@@ -141,7 +141,7 @@ bool generic_supported(int head_dim);
 int generic_max_split(int n_head_kv, int num_cu);
 int generic_rows_per_split(int n_rows, int max_split);
 // Once per handle, its device current: above 64 KiB of dynamic LDS (head_dim
-// above 192) the kernel's limit has to be raised.
+// above 200) the kernel's limit has to be raised.
 hipError_t prepare_generic_decode(int head_dim);
 hipError_t launch_generic_decode(const GenericArgs &a, const RopeRow &rr, hipStream_t s);
 
