@@ -508,11 +508,15 @@ __device__ __attribute__((noinline)) void prefill_fp32(uint64_t args, int work, 
                 auto count = [&](auto is, float add) {
                     floatx16 n{};
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        const float4 v4 = v_at(j);
+                    for (int ks = 0; ks < 2; ++ks) {
+                        half8 c, on;                 // keys 16 ks + 8 (e / 4) + 4 qg + e % 4
 #pragma unroll
-                        for (int e = 0; e < 4; ++e)
-                            n = mfma32f(is(comp(v4, e)) ? 1.f : 0.f, k0 + 8 * j + 4 * qg + e <= qpos ? 1.f : 0.f, n);
+                        for (int e = 0; e < 8; ++e) {
+                            const int j = 2 * ks + e / 4;
+                            c[e] = is(comp(v_at(j), e % 4)) ? (_Float16)1.f : (_Float16)0.f;
+                            on[e] = k0 + 8 * j + 4 * qg + e % 4 <= qpos ? (_Float16)1.f : (_Float16)0.f;
+                        }
+                        n = mfma32h(c, on, n);
                     }
 #pragma unroll
                     for (int r = 0; r < 16; ++r) acc[tt][r] += n[r] > 0.f ? add : 0.f;
