@@ -404,10 +404,10 @@ __device__ __attribute__((noinline)) void prefill_fp32(uint64_t args, int work, 
     for (int tt = 0; tt < NT; ++tt) acc[tt] = floatx16{};
     float m_run = -INFINITY, l_run = 0.f;
     // Tiles: K as chunks of 4 dims [hd / 4][33 keys], V as groups
-    // of 4 keys [8][hd], 16 bytes a unit, and whether V has infinities or NaN.
+    // of 4 keys [8][hd], 16 bytes a unit, and which of +inf, -inf and NaN V has.
     auto write_tile32 = [&](int bo) {
         L.clear_pad();
-        bool odd = false;
+        bool top = false, low = false, nan = false;
 #pragma unroll
         for (int i = 0; i < NUK; ++i) {
             const int u = lane + 64 * i;
@@ -424,7 +424,11 @@ __device__ __attribute__((noinline)) void prefill_fp32(uint64_t args, int work, 
             for (int d = 0; d < VD; ++d) {
                 const float8v x = L.rv[i][d];
 #pragma unroll
-                for (int e = 0; e < 8; ++e) odd |= !(__builtin_fabsf(x[e]) < __builtin_inff());
+                for (int e = 0; e < 8; ++e) {
+                    top |= x[e] == __builtin_inff();
+                    low |= x[e] == -__builtin_inff();
+                    nan |= x[e] != x[e];
+                }
                 unsigned char *dst = lds + bo + kVOff32 + ((4 * (wave >> 1) + (wave & 1)) * HDP + VD * u + d) * 16;
                 if ((HDP / VD) % 64 == 0 || u < HDP / VD) {
                     st4((float *)dst, make_float4(x[0], x[1], x[2], x[3]));
@@ -432,8 +436,9 @@ __device__ __attribute__((noinline)) void prefill_fp32(uint64_t args, int work, 
                 }
             }
         }
-        const int any = __builtin_amdgcn_ballot_w64(odd) != 0;
-        if (lane == 0) ((int *)(lds + bo + kMeta))[8 + wave] = any;
+        const int odd = (__builtin_amdgcn_ballot_w64(top) != 0) | (__builtin_amdgcn_ballot_w64(low) != 0) << 1 |
+                        (__builtin_amdgcn_ballot_w64(nan) != 0) << 2;
+        if (lane == 0) ((int *)(lds + bo + kMeta))[8 + wave] = odd;
     };
 
     auto compute_tile32 = [&](int bo, int t) {
@@ -441,7 +446,7 @@ __device__ __attribute__((noinline)) void prefill_fp32(uint64_t args, int work, 
         if (k0 > L.my_kmax) return;
         const unsigned char *kp = lds + bo + (66 * qg + qi) * 16, *vp = lds + bo + kVOff32 + (qg * HDP + qi) * 16;
         const int4 ov = *(const int4 *)(lds + bo + kMeta + 32);
-        const bool odd = __builtin_amdgcn_readfirstlane(ov.x | ov.y | ov.z | ov.w) != 0;
+        const int odd = __builtin_amdgcn_readfirstlane(ov.x | ov.y | ov.z | ov.w);
         floatx16 s{};
         double sd[EXACT ? 1 : 16];
 #pragma unroll
@@ -521,9 +526,9 @@ __device__ __attribute__((noinline)) void prefill_fp32(uint64_t args, int work, 
 #pragma unroll
                     for (int r = 0; r < 16; ++r) acc[tt][r] += n[r] > 0.f ? add : 0.f;
                 };
-                count([](float x) { return x == __builtin_inff(); }, __builtin_inff());
-                count([](float x) { return x == -__builtin_inff(); }, -__builtin_inff());
-                count([](float x) { return x != x; }, __builtin_nanf(""));
+                if (odd & 1) count([](float x) { return x == __builtin_inff(); }, __builtin_inff());
+                if (odd & 2) count([](float x) { return x == -__builtin_inff(); }, -__builtin_inff());
+                if (odd & 4) count([](float x) { return x != x; }, __builtin_nanf(""));
             }
             __builtin_amdgcn_sched_barrier(0);
         }
