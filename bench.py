@@ -62,14 +62,14 @@ WARM_SECONDS = 0.5             # least decode work ahead of the timed region (st
 # (fetch x 2.0, write x 1.0): decode layer = split + combine kernel, prefill layer =
 # append + prefill + prefill combine kernel.  Re-measure when a kernel changes.
 TRAFFIC_DECODE_BYTES = 19_082_000
-TRAFFIC_PREFILL_BYTES = 141_000_000
+TRAFFIC_PREFILL_BYTES = 140_188_000
 # the same for the matvec leg's dominant launch, ffn_gate + ffn_up of one layer (76.55 MB
 # of weights, activations and outputs algorithmic)
 TRAFFIC_MATVEC_BYTES = {"ffn_gate_q4k+ffn_up_q4k": 80_449_000}
 # the same for the batched matmul leg's dominant launch, ffn_gate + ffn_up of one layer on 64
-# activations (87.17 MB algorithmic), fp16 path: split pre-pass 1.93 MB, main kernel 124.3 MB
-# (the partials of split tiles included), fix-up 35.1 MB
-TRAFFIC_GEMM_BYTES = {"ffn_gate_q4k+ffn_up_q4k": 161_290_000}
+# activations (87.17 MB algorithmic), fp16 path: split pre-pass 1.92 MB, main kernel 125.1 MB
+# (the partials of split tiles included), fix-up 35.0 MB
+TRAFFIC_GEMM_BYTES = {"ffn_gate_q4k+ffn_up_q4k": 161_983_000}
 FP16_MFMA_PEAK_TFLOPS = 2500.0  # MI355X dense fp16 matrix, published
 # prefill attention: every product is three fp16 ones (operands split in two)
 PREFILL_MFMA_PEAK_TFLOPS = round(FP16_MFMA_PEAK_TFLOPS / 3, 1)

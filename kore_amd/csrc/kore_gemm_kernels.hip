@@ -606,10 +606,10 @@ __device__ __forceinline__ void store16(const GemmArgs &a, const GemmMat &mt, in
 // consecutive lanes.  Loaded straight to the lanes that use them, 16 bytes of 32
 // rows at a time, every cache line was asked for up to eight times while its
 // first miss was pending, and the waves stood in line for a third of the kernel.
-// What bounds it: the MFMAs (a block takes a CU 4200 cycles of them, 5000 with the
-// dequantisation between, some 7900 with the copies' issue and the two barriers),
-// and a start of 9000 cycles until the first block's data is there, of runs of 4
-// to 5 blocks.  Whole call, pre-pass and fix-up included, against loads straight
+// What bounds it: of 13.9 thousand cycles per block (7B gate and up, runs of 8
+// blocks, the start until the first block's data is there included) a CU's MFMAs
+// are busy 4.2; the dequantisation stands between them, the copies' issue and two
+// barriers beside them.  Whole call, pre-pass and fix-up included, against loads straight
 // to registers: 18944 x 3584 Q4_K, 64 activations 39.9 -> 38.4 us; 3584 x 3584
 // 23.0 -> 21.8; 3584 x 18944 Q6_K, 19 activations 42.8 -> 40.9; 8960 x 1536 Q4_K,
 // 22 activations 18.7 -> 17.0.

@@ -4,7 +4,8 @@
 //
 //   prefill_kernel          causal attention of a chunk of query rows over the
 //                           cache, both products on fp16 MFMA with every
-//                           operand split into two fp16 parts
+//                           operand split into two or three fp16 parts
+//   prefill_fp32            the same on fp32 MFMA, where the parts would lose bits
 //   prefill_combine_kernel  merge of the key ranges that a query row's work
 //                           was split into
 //
@@ -14,29 +15,33 @@
 // summed in fp32) cost 3 / 16 of the fp32 ones.  The sums take 16 products per
 // fp32 rounding instead of two, and the score's small cross terms are summed
 // first, so the result is nearer to the exact one than the fp32 kernel's was
-// (28/4/128, 2048 rows: 3.9e-7 of the 2-norm against 7.2e-7).  A head_dim that
-// is neither 64 nor 128 ran on VALU with fp64 scores; to lose nothing there a
-// third part holds the last bit (six products) and the scores' 16-dim pieces
-// are summed in fp64 (33/3/96, 700 rows: 2.8e-7 against 4.0e-7; 4/4/140, 175
-// rows: 1.4e-7 against 1.8e-7).
+// (28/4/128, 2048 rows, mean of six draws: 5.0e-7 of the 2-norm against 9.1e-7;
+// 12/2/128, 333 rows at 7001: 6.6e-7 against 1.28e-6).  A head_dim that is neither
+// 64 nor 128 ran on VALU with fp64 scores; to lose nothing there a third part
+// holds the last bit (six products) and the scores' 16-dim pieces are summed in
+// fp64 (33/3/96, 700 rows at 100: 2.4e-7 against 3.9e-7).  A call of a few keys may
+// differ by one rounding of the MFMA's sum either way (one row alone: 1.4e-8, and V
+// itself before).
 //
 // Measured, one layer, against the kernels before (fp32 MFMA; VALU for 33/3/96):
-// 28/4/128 2048 rows 261 -> 141 us (114 -> 213 TFLOP/s), 12/2/128 333 rows at
-// 7001 151 -> 73 us, 33/3/96 700 rows at 100 731 -> 81 us (101 with one
-// workgroup per CU; two parts with fp64 sums 54 us, but 4/4/140 at 2.0e-7).
-// What bounds it now: the MFMAs (39 % of the cycles) and the softmax and split
-// arithmetic (47 %) hardly overlap, since a wave does one after the other.
+// 28/4/128 2048 rows 261 -> 146 us (115 -> 206 TFLOP/s), 12/2/128 333 rows at
+// 7001 151 -> 75 us, 33/3/96 700 rows at 100 730 -> 93 us.  Before the checks that
+// send a tile to prefill_fp32, and the units that follow the weights, these took
+// 141, 72 and 82 us, with wrong results for the data that needs them.
+// What bounds it: MFMAs 27 % of a SIMD's cycles, other vector instructions 29 to 33 %,
+// and a wave does one after the other (39 % of the waves' time waits for an issue).
 //
 // Range.  fp16 holds 2^-24 .. 65504, so every operand is scaled by a power of
 // two (exact) that brings its largest magnitude to 2^13 .. 2^14: a query row
 // by its own, K and V by groups of eight keys, a query's softmax weights by one
 // that follows them.  A value's parts go down to 2^-25, so what a small one loses
 // is 2^-38 of its group's largest.  Where that could be seen in an output (V
-// whose keys, dims, groups or tiles lie far apart in size, or K and q that make
-// a score coarse) or a value is
-// not finite, the workgroup starts again on prefill_fp32, as the fp32 products
-// were (2.5 times the time of this kernel): such values reach exactly the rows
-// that attend them.
+// whose keys, dims, groups or tiles lie far apart in size, or K and q that make a
+// score coarse) or a value is not finite, the workgroup starts again on
+// prefill_fp32, as the fp32 products were: such values reach exactly the rows that
+// attend them.  With one key's V 1e6 times the others' 28/4/128, 2048 rows take
+// 410 us, 33/3/96, 700 rows 118.
+
 #include "kore_attn_kernels.h"
 #include "kore_attn_device.h"
 

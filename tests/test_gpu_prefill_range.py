@@ -2,7 +2,7 @@
 norm: what a row does not attend, or attends with next to no weight, must not cost it precision, and zeros are
 ordinary values.
 
-Bound: ordinary rows of these sizes measure 1e-7 to 4e-7 of their 2-norm (fp32 sums); where a score may be off by
+Bound: ordinary rows of these sizes measure 1e-7 to 5e-7 of their 2-norm (fp32 sums); where a score may be off by
 2^-21 its weight is off by 3.3e-7 more.  1e-6 holds both.
 """
 import numpy as np
