@@ -116,15 +116,16 @@ constexpr int per_cu(int hdp, bool exact) { return hdp <= (exact ? 128 : 96) ? 2
 constexpr int kMfma = 0x8, kDsRead = 0x100;   // __builtin_amdgcn_sched_group_barrier classes
 constexpr int kBK = 32;           // keys per tile
 // Limits of the two- and three-part products.  Weights are scaled so that a
-// tile's largest lies in 2^kTMin .. 2^kTMax (fp16 ends below 2^16; at 2^kTMin its
-// parts still have 24 bits beside V groups of 2^-kSpread), and is put to 2^kTNew
-// where it does not; below 2^kTMin it matters only to an output that is small in
-// the same units: kEnough is 2^22 against the 2^-11 that a lost part is worth
-// (2^-25 times V's 2^14).
-constexpr float kTMax = 15.f, kTMin = 3.f;
+// tile's largest lies in 2^kTMin .. 2^kTMax (fp16 ends below 2^16), and is put to
+// 2^kTNew where it does not; below 2^kTMin it matters only to an output that is
+// small in the same units: kEnough is 2^22 against the 2^-11 that a lost part is
+// worth (2^-25 times V's 2^14).  At 2^kTMin the parts still have 24 bits beside V
+// groups of 2^-kSpread, a spread that tokens whose V differ 50-fold do not reach
+// (28/4/128, 2048 rows: 151 us; with a limit of 2^-3 459, in the fp32 loop).
+constexpr float kTMax = 15.f, kTMin = 8.f;
 constexpr int kTNew = 11;
 constexpr float kEnough = 0x1p22f;
-constexpr int kSpread = 3;        // log2 of the spread of V's group scales in a tile
+constexpr int kSpread = 6;        // log2 of the spread of V's group scales in a tile
 constexpr int kRange = 40;        // ... and over a workgroup's tiles (exponents stay in fp32's range)
 constexpr int kNone = 1 << 20;    // a unit before any key (pow2 drops it)
 

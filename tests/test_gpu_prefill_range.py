@@ -180,3 +180,30 @@ def test_large_channel_of_q_that_k_lacks(nh, nkv, hd):
     k[:, ::hd] = 0.0
     k[:, hd // 2::hd] = 0.0
     check(q, k, v, 40, nh, nkv, hd)
+
+
+@pytest.mark.parametrize("nh,nkv,hd", GEOMETRIES)
+@pytest.mark.parametrize("spread", [3, 8])
+def test_v_of_many_sizes(nh, nkv, hd, spread):
+    """Every key's V its own size, and rows that attend a few keys, the smallest ones among them."""
+    q, k, v = inputs(96, 100, nh, nkv, hd, 23)
+    v *= np.exp2(np.random.default_rng(24).uniform(-spread, spread, (196, 1))).astype(np.float32)
+    q *= np.float32(4.0)
+    # scores of up to 4 * 4 sigma / ln 2, each and their differences rounded in fp32
+    check(q, k, v, 100, nh, nkv, hd, tol=1e-6 + 24 * 2.0 ** -22 * 0.69)
+
+
+@pytest.mark.parametrize("nh,nkv,hd", GEOMETRIES)
+@pytest.mark.parametrize("key", [0, 45])
+@pytest.mark.parametrize("drop", [8.0, 16.0, 24.0])
+def test_sink_with_a_small_v(nh, nkv, hd, key, drop):
+    """A key takes nearly all the weight and its V is 2^-9 of the others'."""
+    q, k, v = inputs(40, 100, nh, nkv, hd, 25)
+    q *= np.float32(0.2)
+    q[:, ::hd] = 8.0
+    k[:, ::hd] = 0.0
+    k[key] = 0.0
+    k[key, ::hd] = np.float32(drop * np.sqrt(hd) / 8.0)
+    q, k = unrotate(q, np.arange(100, 140), hd), unrotate(k, np.arange(140), hd)
+    v[key] *= np.float32(2.0 ** -9)
+    check(q, k, v, 100, nh, nkv, hd, tol=1e-6 + drop * 1.45 * 2.0 ** -23)
